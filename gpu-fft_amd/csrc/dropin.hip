@@ -1,7 +1,7 @@
 // Drop-in entry points: GPU_FFT (C_C and R_R), GPU_FFNT and GPU_Special_FFT
 // of the reference (src/lib/fft.cu:517-725, 928-1007, 1386-1515), as C ABI.
 // Each call validates on the host, then enqueues one launch per pass on
-// cfg->stream (one launch in total up to 2^12 double / 2^13 float points).
+// cfg->stream (one launch in total up to 2^13 points).
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -250,37 +250,14 @@ int special_split(void* inout, const void* table, const gpufft_config* cfg, int 
     return run_transform<float>(mode, n, batch, 0, (const cplx<float>*)table, io, st, who);
 }
 
-// CKKS slot <-> coefficient steps around the special FFT.  l = 2^n slots,
-// ring N = 2l: coefficient i pairs with slot-transform entry bitrev(i) (the
-// special inverse leaves its output bit-reversed, the special forward wants
-// its input bit-reversed; fft.cu:727-926), real parts give m[0..l), imaginary
-// parts m[l..2l).
-__global__ void ckks_round_kernel(const cplx<double>* u, long long* m, int n, long long total,
-                                  double delta)
-{
-    const long long t = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (t >= total) return;
-    const long long l = 1LL << n;
-    const long long b = t >> n;
-    const int i = (int)(t & (l - 1));
-    const int br = (int)(__brev((unsigned)i) >> (32 - n));
-    const cplx<double> z = u[b * l + br];
-    m[2 * b * l + i] = llround(z.x * delta);
-    m[2 * b * l + i + l] = llround(z.y * delta);
-}
-
-__global__ void ckks_unround_kernel(const long long* m, cplx<double>* v, int n, long long total,
-                                    double delta)
-{
-    const long long t = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (t >= total) return;
-    const long long l = 1LL << n;
-    const long long b = t >> n;
-    const int i = (int)(t & (l - 1));
-    const int br = (int)(__brev((unsigned)i) >> (32 - n));
-    v[b * l + br] = mk<double>((double)m[2 * b * l + i] / delta, (double)m[2 * b * l + i + l] / delta);
-}
-
+// CKKS slot <-> coefficient forms of the special FFT.  l = 2^n slots, ring
+// N = 2l: coefficient i pairs with slot-transform entry bitrev(i) (the special
+// inverse leaves its output bit-reversed, the special forward wants its input
+// bit-reversed; fft.cu:727-926), real parts give m[0..l), imaginary parts
+// m[l..2l).  The conversion and the reordering are the last pass's store
+// (encode) and the first pass's load (decode): 432 us for 512 x 2^15 slots
+// there and back.  As passes of their own, with one uncoalesced side each,
+// they took 297 us beside 534 us of transform passes.
 int check_ckks(int n_power, double delta, int batch, const char* who)
 {
     if (n_power < GPUFFT_MIN_N_POWER || n_power > GPUFFT_MAX_N_POWER)
@@ -302,20 +279,15 @@ int ckks_encode(const void* slots, int64_t* coeffs, const void* inv_table, int n
     io.lk = LD_CPLX;
     io.src = slots;
     io.src_stride = L;
-    io.sk = ST_CPLX;
-    io.dst = work;
-    io.dst_stride = L;
+    io.sk = ST_CKKS;
+    io.dst = coeffs;
+    io.dst_stride = 2 * L;
     io.work = (cplx<double>*)work;
     io.do_scale = true;
     io.scale = mk<double>(1.0 / (double)L, 0.0);
-    if (int s = run_transform<double>(MODE_SPE_INV, n_power, batch, 0, (const cplx<double>*)inv_table,
-                                      io, st, who))
-        return s;
-    const long long total = (long long)batch << n_power;
-    hipLaunchKernelGGL(ckks_round_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st,
-                       (const cplx<double>*)work, (long long*)coeffs, n_power, total, delta);
-    GFA_CHECK_LAUNCH(who);
-    return ok();
+    io.delta = delta;
+    return run_transform<double>(MODE_SPE_INV, n_power, batch, 0, (const cplx<double>*)inv_table, io,
+                                 st, who);
 }
 
 int ckks_decode(const int64_t* coeffs, void* slots, const void* table, int n_power, double delta,
@@ -326,19 +298,16 @@ int ckks_decode(const int64_t* coeffs, void* slots, const void* table, int n_pow
         return fail(GPUFFT_ERR_NULL_POINTER, std::string(who) + ": NULL buffer");
     const long long L = 1LL << n_power;
     hipStream_t st = (hipStream_t)stream;
-    const long long total = (long long)batch << n_power;
-    hipLaunchKernelGGL(ckks_unround_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st,
-                       (const long long*)coeffs, (cplx<double>*)slots, n_power, total, delta);
-    GFA_CHECK_LAUNCH(who);
     cplx<double>* x = (cplx<double>*)slots;
     TransformIO<double> io{};
-    io.lk = LD_CPLX;
-    io.src = x;
-    io.src_stride = L;
+    io.lk = LD_CKKS;
+    io.src = coeffs;
+    io.src_stride = 2 * L;
     io.sk = ST_CPLX;
     io.dst = x;
     io.dst_stride = L;
     io.work = x;
+    io.delta = delta;
     return run_transform<double>(MODE_SPE_FWD, n_power, batch, 0, (const cplx<double>*)table, io, st,
                                  who);
 }

@@ -474,7 +474,7 @@ __global__ __launch_bounds__((1 << S) >> E) void product_sub_kernel(ProdArgs<T> 
         asm volatile("" : "+v"(t));
         __syncthreads();
         load_sub<T, S, SB, E, PL, HB>(lds, a, xb, tws, a.wb, jb, KB, a.ob, 0, false, C, q, t);
-        run_steps_ct<T, MODE_STD_FWD, E, NT, S, RB, FS0, NST - 1, true>(lds, pf, g, t, a.wc);
+        run_steps_ct<T, MODE_STD_FWD, E, NT, S, RB, FS0, NST - 1>(lds, pf, g, t, a.wc);
         last_forward_step<T, E, RB, NT>(lds, pf, g, t, breg, a.wc);
         for (int ia = 0; ia < KA; ia++) {
             int u = tid;
@@ -485,7 +485,7 @@ __global__ __launch_bounds__((1 << S) >> E) void product_sub_kernel(ProdArgs<T> 
             if (!jl) {
                 load_sub<T, S, SB, E, PL, HB>(lds, a, xa, tws, a.wa, ia, a.ka, a.oa,
                                               a.ca ? (1 << a.ca) : 0, false, C, q, u);
-                run_steps_ct<T, MODE_STD_FWD, E, NT, S, RB, FS0, NST - 1, true>(lds, pf, g, u,
+                run_steps_ct<T, MODE_STD_FWD, E, NT, S, RB, FS0, NST - 1>(lds, pf, g, u,
                                                                                a.wc);
             }
             // last forward step, product, first inverse step: in registers,
@@ -509,7 +509,7 @@ __global__ __launch_bounds__((1 << S) >> E) void product_sub_kernel(ProdArgs<T> 
 #pragma unroll
                 for (int j = 0; j < (1 << RB); j++) lds[swz(rbase | j)] = v[j];
             }
-            run_steps_ct<T, MODE_STD_INV, E, NT, S, RB, 1, IEND, true>(lds, pinv, gi, u, a.wci);
+            run_steps_ct<T, MODE_STD_INV, E, NT, S, RB, 1, IEND>(lds, pinv, gi, u, a.wci);
             // element i of this thread: position u + i NT; the top step joins
             // elements i + m EPT/2^HB (positions c + m 2^(S-HB))
             constexpr int NP = 1 << HB;

@@ -99,7 +99,7 @@ __global__ __launch_bounds__((1 << S) >> E) void fwd_sub_kernel(OneArgs<T> o)
     const rsrc_t xa = make_rsrc(reinterpret_cast<const T*>(o.src) + t * o.src_stride);
     __syncthreads();
     load_sub<T, S, SB, E, PL, HB>(lds, a, xa, tws, 0, 0, 1, 0, 0, false, C, q, tid);
-    run_steps_ct<T, MODE_STD_FWD, E, NT, S, RB, FS0, NST, true, true>(lds, pf, g, tid, o.tab);
+    run_steps_ct<T, MODE_STD_FWD, E, NT, S, RB, FS0, NST, true>(lds, pf, g, tid, o.tab);
     cplx<T>* dst = reinterpret_cast<cplx<T>*>(o.dst) + t * o.dst_stride + ((long long)q << S);
 #pragma unroll 4
     for (int i = 0; i < EPT; i++) {
@@ -153,7 +153,7 @@ __global__ __launch_bounds__((1 << S) >> E) void inv_local_kernel(OneArgs<T> o)
     g.K = S;
     g.logC = 0;
     g.tab = make_rsrc(o.tab);
-    run_steps_ct<T, MODE_STD_INV, E, NT, S, RB, 0, IEND, true, true>(lds, pi, g, tid, o.tab);
+    run_steps_ct<T, MODE_STD_INV, E, NT, S, RB, 0, IEND, true>(lds, pi, g, tid, o.tab);
     ProdArgs<T> a{};
     a.n = o.n;
     a.S = S;

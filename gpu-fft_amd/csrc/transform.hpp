@@ -3,59 +3,48 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <cmath>
 #include <vector>
 
 #include "engine.hpp"
 #include "oneshot.hpp"
+#include "passes.hpp"
 #include "status.hpp"
 
 namespace gfa {
 
-// Tile geometry per element type: 2^LOGT elements of 16 bytes (double) or
-// 8 bytes (float) = 64 KiB of LDS, 16 elements per thread, 256 / 512 threads.
-template <typename T> struct TileCfg;
-template <> struct TileCfg<double> {
-    static constexpr int LOGT = 12;
-    static constexpr int E = 4;
-};
-template <> struct TileCfg<float> {
-    static constexpr int LOGT = 13;
-    static constexpr int E = 4;
-};
-
 struct PassPlan {
-    int blo, K, logC, logBT;
+    bool col;
+    int blo, K;
 };
 
-// Splits the n position bits into passes of at most LOGT bits.  The pass
-// that reaches bit 0 takes LOGT bits (contiguous tiles); the others take at
-// most LOGT-4 bits so that every tile row is at least 16 contiguous elements.
-// Descending modes run the top bits first, ascending modes bit 0 first.
-inline std::vector<PassPlan> plan_passes(int n, int LOGT, bool descending)
+// Splits the n position bits into passes, ascending: one row pass over bits
+// [0, K0) and column passes above it (pass.hpp).  One row pass up to 13 bits;
+// two passes to 2^24: 8 column bits keep 128-byte column rows and two radix
+// steps, and the row pass takes the rest, up to the 12 bits of the 2^12 tile;
+// beyond 2^20 the column pass grows too.  (FP64, 2^23 points, batch 1: 100 us
+// in 2 passes, 5.4 TB/s, against 197 us in 3 passes of at most 12 + 8 bits.)
+// reversed: the CKKS passes read or write the row pass's tile in natural
+// order, which needs 2^(12-K0) >= 16 blocks for 128-byte runs, so K0 <= 8.
+inline std::vector<PassPlan> plan_passes(int n, bool descending, bool reversed)
 {
     std::vector<PassPlan> p;
-    if (n <= LOGT) {
-        p.push_back({0, n, 0, LOGT - n});
+    if (n <= PASS_ROW_MAX) {
+        p.push_back({false, 0, n});
         return p;
     }
-    int rest = n - LOGT;
-    int maxk = LOGT - 4;
-    int cnt = (rest + maxk - 1) / maxk;
-    std::vector<int> ks;
-    for (int i = 0; i < cnt; i++) ks.push_back(rest / cnt + (i < rest % cnt ? 1 : 0));
-    // ascending order of bits: [0,LOGT), then the chunks upward
-    std::vector<PassPlan> asc;
-    asc.push_back({0, LOGT, 0, 0});
-    int b = LOGT;
-    for (int k : ks) {
-        asc.push_back({b, k, LOGT - k, 0});
-        b += k;
-    }
-    if (descending) {
-        for (int i = (int)asc.size() - 1; i >= 0; i--) p.push_back(asc[i]);
+    int c = n <= 16 ? n - n / 2 : n <= 20 ? 8 : n - 13 < 9 ? 9 : n - 13;
+    if (reversed) c = n - 8;
+    if (c <= PASS_COL_MAX) {
+        p.push_back({false, 0, n - c});
+        p.push_back({true, n - c, c});
     } else {
-        p = asc;
+        p.push_back({false, 0, n - c});
+        p.push_back({true, n - c, c / 2});
+        p.push_back({true, n - c + c / 2, c - c / 2});
     }
+    if (descending) std::reverse(p.begin(), p.end());
     return p;
 }
 
@@ -73,78 +62,27 @@ template <typename T> struct TransformIO {
     cplx<T>* work;          // complex [batch][2^n] buffer for intermediate passes
     bool do_scale;
     cplx<T> scale;
+    double delta;           // LD_CKKS, ST_CKKS
 };
-
-template <typename T>
-using PassFn = void (*)(PassArgs<T>);
-
-template <typename T, int MODE, int LK, int SK, int BIG> inline PassFn<T> pass_fn()
-{
-    return &pass_kernel<T, MODE, TileCfg<T>::LOGT + BIG, TileCfg<T>::E, LK, SK>;
-}
-
-// Kernel for (mode, load kind, store kind); nullptr for combinations no
-// operation uses.  BIG = 1: tile of 2^(LOGT+1) elements (twice the LDS and
-// threads), so that a transform of exactly 2^(LOGT+1) points is one pass.
-template <typename T, int BIG> PassFn<T> select_pass(int mode, int lk, int sk)
-{
-#define GFA_SEL(M, L, S) \
-    if (mode == M && lk == L && sk == S) return pass_fn<T, M, L, S, BIG>();
-    GFA_SEL(MODE_STD_FWD, LD_CPLX, ST_CPLX)
-    GFA_SEL(MODE_STD_FWD, LD_REAL, ST_CPLX)
-    GFA_SEL(MODE_STD_FWD, LD_FOLD, ST_CPLX)
-    GFA_SEL(MODE_STD_INV, LD_CPLX, ST_CPLX)
-    GFA_SEL(MODE_STD_INV, LD_MUL, ST_CPLX)
-    GFA_SEL(MODE_STD_INV, LD_CPLX, ST_REAL)
-    GFA_SEL(MODE_STD_INV, LD_MUL, ST_REAL)
-    GFA_SEL(MODE_STD_INV, LD_CPLX, ST_UNFOLD)
-    GFA_SEL(MODE_STD_INV, LD_RR_PACK, ST_CPLX)
-    GFA_SEL(MODE_STD_INV, LD_MUL, ST_UNFOLD)
-    GFA_SEL(MODE_SPE_FWD, LD_CPLX, ST_CPLX)
-    GFA_SEL(MODE_SPE_INV, LD_CPLX, ST_CPLX)
-    if constexpr (sizeof(T) == 4) {
-        GFA_SEL(MODE_SPE_FWD, LD_SPLIT_HI, ST_CPLX)
-        GFA_SEL(MODE_SPE_FWD, LD_SPLIT_LO, ST_CPLX)
-        GFA_SEL(MODE_SPE_FWD, LD_SPLIT_LO, ST_SUM_F64)
-        GFA_SEL(MODE_SPE_FWD, LD_CPLX, ST_SUM_F64)
-        GFA_SEL(MODE_SPE_INV, LD_SPLIT_HI, ST_CPLX)
-        GFA_SEL(MODE_SPE_INV, LD_SPLIT_LO, ST_CPLX)
-        GFA_SEL(MODE_SPE_INV, LD_SPLIT_LO, ST_SUM_F64)
-        GFA_SEL(MODE_SPE_INV, LD_CPLX, ST_SUM_F64)
-    }
-#undef GFA_SEL
-    return nullptr;
-}
 
 // Launches every pass of one transform of length 2^n over `batch` transforms.
 template <typename T>
 int run_transform(int mode, int n, int batch, int nega, const cplx<T>* tab,
                   const TransformIO<T>& io, hipStream_t stream, const char* who)
 {
-    constexpr int LOGT0 = TileCfg<T>::LOGT;
-    // double, n = LOGT0 + 1: one pass over a double-size tile (128 KiB of LDS,
-    // 512 threads) instead of two passes (for float the doubled tile would
-    // need 1024 threads, whose 128-register budget spills)
-    const bool big = sizeof(T) == 8 && n == LOGT0 + 1;
-    const int LOGT = big ? LOGT0 + 1 : LOGT0;
-    const int NT = (1 << LOGT) >> TileCfg<T>::E;
-    std::vector<PassPlan> plan = plan_passes(n, LOGT, mode_descending(mode));
+    const bool reversed = io.lk == LD_CKKS || io.sk == ST_CKKS;
+    const std::vector<PassPlan> plan = plan_passes(n, mode_descending(mode), reversed);
     const long long L = 1LL << n;
     for (size_t i = 0; i < plan.size(); i++) {
         const bool first = (i == 0), last = (i + 1 == plan.size());
         const PassPlan& pp = plan[i];
-        PassArgs<T> a{};
+        RadixArgs<T> a{};
         a.n = n;
         a.blo = pp.blo;
-        a.K = pp.K;
-        a.logC = pp.logC;
-        a.logBT = pp.logBT;
         a.batch = batch;
         a.nega = nega;
         a.tab = tab;
         int lk = LD_CPLX, sk = ST_CPLX;
-        a.nt_in = first ? 1 : 0;
-        a.nt_out = last ? 1 : 0;
         if (first) {
             lk = io.lk;
             a.src = io.src;
@@ -166,15 +104,19 @@ int run_transform(int mode, int n, int batch, int nega, const cplx<T>* tab,
             a.dst = io.work;
             a.dst_stride = L;
         }
-        PassFn<T> fn = select_pass<T, 0>(mode, lk, sk);
-        if constexpr (sizeof(T) == 8)
-            if (big) fn = select_pass<T, 1>(mode, lk, sk);
+        a.delta = io.delta;
+        int e2 = 0;
+        if (io.delta > 0 && std::frexp(io.delta, &e2) == 0.5 && std::isfinite(1.0 / io.delta))
+            a.inv_delta = 1.0 / io.delta;
+        RadixFn<T> fn = mode == MODE_STD_FWD ? pass_std_fwd<T>(pp.col, pp.K, lk, sk)
+                      : mode == MODE_STD_INV ? pass_std_inv<T>(pp.col, pp.K, lk, sk)
+                      : mode == MODE_SPE_FWD ? pass_spe_fwd<T>(pp.col, pp.K, lk, sk)
+                                             : pass_spe_inv<T>(pp.col, pp.K, lk, sk);
         if (!fn) return fail(GPUFFT_ERR_UNSUPPORTED, std::string(who) + ": no kernel for this pass");
-        long long tiles = ((long long)batch << n) >> LOGT;
-        if (pp.logBT > 0) tiles = ((long long)batch + (1LL << pp.logBT) - 1) >> pp.logBT;
-        if (tiles <= 0) tiles = 1;
+        const int LT = pass_tile<T>(pp.col, pp.K);
+        const long long tiles = (((long long)batch << n) + (1LL << LT) - 1) >> LT;
         if (tiles > 0x7fffffffLL) return fail(GPUFFT_ERR_INVALID_ARGUMENT, std::string(who) + ": batch too large");
-        hipLaunchKernelGGL(fn, dim3((unsigned)tiles), dim3(NT), 0, stream, a);
+        hipLaunchKernelGGL(fn, dim3((unsigned)tiles), dim3((1 << LT) >> PASS_E), 0, stream, a);
         GFA_CHECK_LAUNCH(who);
     }
     return ok();
