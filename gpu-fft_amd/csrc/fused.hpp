@@ -1,4 +1,6 @@
-// Fused polynomial-product kernels for gfx950.
+// Fused FP32-split polynomial products for gfx950, and the gather and step
+// helpers they share with the batched kernel and the one-launch transforms
+// (the FP64 products are product.hpp).
 //
 // A product of two length-2^n transforms (FFNT folding: n = log2(N) - 1) is
 // computed by 2^SB workgroups per product.  Workgroup q owns the sub-problem
@@ -11,16 +13,14 @@
 //      SB-stage network in registers (the other workgroups of the product
 //      read the same inputs, which the XCD-aware block order keeps in L2),
 //   2. runs the S forward stages of operand b in LDS and keeps the result in
-//      registers, then does the same for operand a (or each limb of a),
+//      registers, then does the same for each limb of a,
 //   3. multiplies in registers, inverse-transforms in LDS and writes the
 //      2^S partial results to a scratch buffer.
-// A second, streaming pass applies the top SB inverse stages, the scale, the
-// untwist and the unfold (FP64: f64_combine_kernel; FP32 limbs:
-// limb_combine_kernel, which also rounds each limb product and recombines
-// them in int64).  With SB = 0 an FP64 product is one workgroup and writes the
-// output directly.  The scratch is written and read with streaming hints: it
-// is used once, and must not displace the operand lines that the sibling
-// workgroups of a product re-read from L2.
+// A second, streaming pass (limb_combine_kernel) applies the top SB inverse
+// stages, the scale, the untwist and the unfold, rounds each limb product and
+// recombines them in int64.  The scratch is written and read with streaming
+// hints: it is used once, and must not displace the operand lines that the
+// sibling workgroups of a product re-read from L2.
 //
 // The stage/twiddle semantics are those of the reference GPU_FFNT
 // (src/lib/fft.cu:1013-1384) and GPU_FFT (fft.cu:11-260): bit-reversed
@@ -52,17 +52,13 @@ template <typename T> struct ProdArgs {
     const void* a;
     const void* b;
     long long in_stride;   // input elements per product
-    cplx<T>* scratch;      // [batch][limb products][L] partial results (SB > 0)
-    T* out;                // direct output (SB == 0, PL_FOLD)
-    long long out_stride;
-    cplx<T> scale;
+    cplx<T>* scratch;      // [batch][limb products][L] partial results
     int wa, ka, wb, kb;    // limb split of a and b (PL_FOLD_LIMB)
     long long oa, ob;      // digit offsets: sum_{k < K-1} 2^(w-1) 2^(w k)
     int ca;                // PL_FOLD_LIMB: a is split as a - 2^ca (0: as is); the
                            // product then gains the limb 2^ca J b (J = all ones),
                            // run after the ka digit limbs
     const cplx<T>* jspec;  // forward FFNT spectrum of J (L entries, bit-reversed order)
-    int* arrive;           // per-product arrival counters (in-kernel combine)
 };
 
 // Balanced base-2^w digit i of x = v - center, v an int32 (digits d_0 ..
@@ -361,54 +357,7 @@ __device__ __forceinline__ void last_forward_step(const cplx<T>* lds, const Pass
     }
 }
 
-// Top SB Gentleman-Sande stages (bits S .. n-1) of one whole product from
-// its 2^SB sub-problem results in scratch, then scale, untwist and unfold:
-// out[P] = Re, out[P + L] = Im (reference InverseFFNTCoreUnique,
-// src/lib/fft.cu:1298-1384).  Run by the last workgroup of the product.
-template <typename T, int S, int SB, int NT>
-__device__ __forceinline__ void combine_product(const ProdArgs<T>& a, long long p, int tid)
-{
-    constexpr int Q = 1 << SB;
-    const int L = 1 << a.n;
-    const rsrc_t src = make_rsrc(a.scratch + p * (long long)L);
-    const rsrc_t ut = make_rsrc(a.untwist);
-    T* o = a.out + p * a.out_stride;
-    // stage i, pair (j0, j0 + 2^i): twiddle itab[(j0 2^S + c) >> (S + i + 1)] = itab[j0 >> (i+1)]
-    cplx<T> w[Q / 2];
-#pragma unroll
-    for (int m = 0; m < Q / 2; m++) w[m] = a.itab[m];
-#pragma unroll 2
-    for (int c = tid; c < (1 << S); c += NT) {
-        cplx<T> y[Q];
-#pragma unroll
-        for (int j = 0; j < Q; j++) y[j] = bldc<T>(src, (j << S) | c);
-#pragma unroll
-        for (int i = 0; i < SB; i++) {
-#pragma unroll
-            for (int j0 = 0; j0 < Q; j0++) {
-                if (j0 & (1 << i)) continue;
-                const int j1 = j0 | (1 << i);
-                const cplx<T> U = y[j0], V = y[j1];
-                y[j0] = U + V;
-                y[j1] = (U - V) * w[j0 >> (i + 1)];
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < Q; j++) {
-            const int P = (j << S) | c;
-            const cplx<T> z = (y[j] * a.scale) * bldc<T>(ut, P);
-            o[P] = z.x;
-            o[P + L] = z.y;
-        }
-    }
-}
-
-// CMB (FP64, SB > 0): the combine runs inside this kernel.  Each workgroup
-// publishes its sub-problem result (agent-scope release) and counts itself
-// in arrive[p]; the workgroup that arrives last acquires, combines the whole
-// product and resets arrive[p] to 0 for the next launch.  No workgroup waits
-// for another.
-template <typename T, int S, int SB, int E, int PL, int RB, bool CMB = false>
+template <typename T, int S, int SB, int E, int PL, int RB>
 __global__ __launch_bounds__((1 << S) >> E) void product_sub_kernel(ProdArgs<T> a)
 {
     constexpr int TILE = 1 << S;
@@ -449,14 +398,9 @@ __global__ __launch_bounds__((1 << S) >> E) void product_sub_kernel(ProdArgs<T> 
     const int nprod = nla * a.kb;
     const long long L = 1LL << a.n;
 
-    const rsrc_t xa = make_rsrc(reinterpret_cast<const char*>(a.a) +
-                                p * a.in_stride * (PL == PL_FOLD ? (long long)sizeof(T) : 4LL));
-    const rsrc_t xb = make_rsrc(reinterpret_cast<const char*>(a.b) +
-                                p * a.in_stride * (PL == PL_FOLD ? (long long)sizeof(T) : 4LL));
+    const rsrc_t xa = make_rsrc(reinterpret_cast<const int*>(a.a) + p * a.in_stride);
+    const rsrc_t xb = make_rsrc(reinterpret_cast<const int*>(a.b) + p * a.in_stride);
     fill_twist_split<T, S>(tws, a.twist, tid, NT);  // visible after the first barrier below
-    // compile-time single limb for the FP64 form
-    const int KA = PL == PL_FOLD ? 1 : nla;
-    const int KB = PL == PL_FOLD ? 1 : a.kb;
 
     cplx<T> C[Q];
     top_row_coeffs<T, SB>(a, q, C);
@@ -467,21 +411,21 @@ __global__ __launch_bounds__((1 << S) >> E) void product_sub_kernel(ProdArgs<T> 
     constexpr int IEND = HB ? NST - 1 : NST;  // end of the inverse steps through LDS
 
     cplx<T> breg[EPT];
-    for (int jb = 0; jb < KB; jb++) {
+    for (int jb = 0; jb < a.kb; jb++) {
         // an opaque copy of tid per iteration keeps the address arithmetic of
         // the loop body inside the loop (hoisted, it would hold registers)
         int t = tid;
         asm volatile("" : "+v"(t));
         __syncthreads();
-        load_sub<T, S, SB, E, PL, HB>(lds, a, xb, tws, a.wb, jb, KB, a.ob, 0, false, C, q, t);
+        load_sub<T, S, SB, E, PL, HB>(lds, a, xb, tws, a.wb, jb, a.kb, a.ob, 0, false, C, q, t);
         run_steps_ct<T, MODE_STD_FWD, E, NT, S, RB, FS0, NST - 1>(lds, pf, g, t, a.wc);
         last_forward_step<T, E, RB, NT>(lds, pf, g, t, breg, a.wc);
-        for (int ia = 0; ia < KA; ia++) {
+        for (int ia = 0; ia < nla; ia++) {
             int u = tid;
             asm volatile("" : "+v"(u));
             __syncthreads();
             // the J limb (ia == ka) needs no transform: its spectrum is a.jspec
-            const bool jl = PL != PL_FOLD && ia >= a.ka;
+            const bool jl = ia >= a.ka;
             if (!jl) {
                 load_sub<T, S, SB, E, PL, HB>(lds, a, xa, tws, a.wa, ia, a.ka, a.oa,
                                               a.ca ? (1 << a.ca) : 0, false, C, q, u);
@@ -514,58 +458,19 @@ __global__ __launch_bounds__((1 << S) >> E) void product_sub_kernel(ProdArgs<T> 
             // elements i + m EPT/2^HB (positions c + m 2^(S-HB))
             constexpr int NP = 1 << HB;
             constexpr int NI = EPT / NP;
-            if constexpr (SB == 0 && PL == PL_FOLD) {
-                // whole product in this workgroup: scale, untwist, unfold
-                T* o = a.out + p * a.out_stride;
-                const rsrc_t utw = make_rsrc(a.untwist);
+            cplx<T>* dst = a.scratch + (p * nprod + ia * a.kb + jb) * L + ((long long)q << S);
 #pragma unroll 2
-                for (int i = 0; i < NI; i++) {
-                    const int c = u + i * NT;
-                    cplx<T> z[NP];
+            for (int i = 0; i < NI; i++) {
+                const int c = u + i * NT;
+                cplx<T> z[NP];
 #pragma unroll
-                    for (int m = 0; m < NP; m++) z[m] = lds[swz(c + (m << (S - HB)))];
-                    if constexpr (HB > 0) top_gs<T, S, HB>(z, a, q);
+                for (int m = 0; m < NP; m++) z[m] = lds[swz(c + (m << (S - HB)))];
+                if constexpr (HB > 0) top_gs<T, S, HB>(z, a, q);
 #pragma unroll
-                    for (int m = 0; m < NP; m++) {
-                        const int cm = c + (m << (S - HB));
-                        const cplx<T> r = (z[m] * a.scale) * bldc<T>(utw, cm);
-                        o[cm] = r.x;
-                        o[cm + L] = r.y;
-                    }
-                }
-            } else {
-                cplx<T>* dst = a.scratch + (p * nprod + ia * KB + jb) * L + ((long long)q << S);
-#pragma unroll 2
-                for (int i = 0; i < NI; i++) {
-                    const int c = u + i * NT;
-                    cplx<T> z[NP];
-#pragma unroll
-                    for (int m = 0; m < NP; m++) z[m] = lds[swz(c + (m << (S - HB)))];
-                    if constexpr (HB > 0) top_gs<T, S, HB>(z, a, q);
-#pragma unroll
-                    for (int m = 0; m < NP; m++) stc_nt(dst + c + (m << (S - HB)), z[m]);
-                }
+                for (int m = 0; m < NP; m++) stc_nt(dst + c + (m << (S - HB)), z[m]);
             }
         }
     }
-    if constexpr (CMB && SB > 0 && PL == PL_FOLD) {
-        __shared__ int sh_last;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        __syncthreads();
-        if (tid == 0) {
-            const int prev = __hip_atomic_fetch_add(a.arrive + p, 1, __ATOMIC_ACQ_REL,
-                                                    __HIP_MEMORY_SCOPE_AGENT);
-            sh_last = prev == Q - 1;
-        }
-        __syncthreads();
-        if (sh_last) {
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-            combine_product<T, S, SB, NT>(a, p, tid);
-            if (tid == 0)
-                __hip_atomic_store(a.arrive + p, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-    }
-    (void)Q;
 }
 
 // FP32 limb products -> int64: top SB inverse stages, scale, untwist, unfold,
@@ -573,79 +478,6 @@ __global__ __launch_bounds__((1 << S) >> E) void product_sub_kernel(ProdArgs<T> 
 // One thread per (product, sub-problem position c).  err (optional) receives
 // per product the largest |x - rint(x)| (as double bits) and the sum of
 // squares over all limb outputs.
-// FP64 products: top SB Gentleman-Sande stages (bits S .. n-1), scale,
-// untwist and unfold (reference InverseFFNTCoreUnique, src/lib/fft.cu:
-// 1298-1384).  A workgroup takes 512 consecutive columns of one product
-// (S >= 9), each thread the columns c and c + 256: the lanes of every load
-// read consecutive 16-byte scratch entries and the lanes of every store
-// write consecutive doubles.  untwist[P] = untwist[P & ~127] *
-// untwist[P & 127] from LDS (the table is exp(-2 pi i P / 2N),
-// multiplicative in P).
-struct F64CombineArgs {
-    int n, S, batch;
-    const cplx<double>* scratch;  // [batch][2^n]
-    const cplx<double>* itab;
-    const cplx<double>* untwist;
-    double scale;
-    double* out;                  // [batch][out_stride]
-    long long out_stride;
-};
-
-constexpr int F64C_MAX_N = 16;  // 2^(16-7) entries in the LDS high-part table
-
-template <int SB>
-__global__ __launch_bounds__(256) void f64_combine_kernel(F64CombineArgs a)
-{
-    constexpr int Q = 1 << SB;
-    __shared__ cplx<double> ut[128 + (1 << (F64C_MAX_N - 7))];
-    const int tid = threadIdx.x;
-    const int nhi = 1 << (a.n - 7);
-    for (int i = tid; i < 128 + nhi; i += 256)
-        ut[i] = i < 128 ? a.untwist[i] : a.untwist[(i - 128) << 7];
-    __syncthreads();
-    const long long g0 = (long long)blockIdx.x * 512;
-    const long long p = g0 >> a.S;
-    const int c = (int)(g0 & ((1LL << a.S) - 1)) + tid;
-    if (p >= a.batch) return;
-    const long long L = 1LL << a.n;
-    const cplx<double>* src = a.scratch + p * L;
-    cplx<double> w[Q > 1 ? Q / 2 : 1];
-#pragma unroll
-    for (int m = 0; m < Q / 2; m++) w[m] = a.itab[m];
-    cplx<double> y[2][Q];
-#pragma unroll
-    for (int j = 0; j < Q; j++) {
-        y[0][j] = ldc_nt(src + ((long long)j << a.S) + c);
-        y[1][j] = ldc_nt(src + ((long long)j << a.S) + c + 256);
-    }
-    double* o = a.out + p * a.out_stride;
-#pragma unroll
-    for (int v = 0; v < 2; v++) {
-#pragma unroll
-        for (int i = 0; i < SB; i++) {
-#pragma unroll
-            for (int j0 = 0; j0 < Q; j0++) {
-                if (j0 & (1 << i)) continue;
-                const int j1 = j0 | (1 << i);
-                const cplx<double> U = y[v][j0], V = y[v][j1];
-                y[v][j0] = U + V;
-                y[v][j1] = (U - V) * w[j0 >> (i + 1)];
-            }
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < Q; j++) {
-#pragma unroll
-        for (int v = 0; v < 2; v++) {
-            const int P = (j << a.S) | (c + 256 * v);
-            const cplx<double> z = mk<double>(y[v][j].x * a.scale, y[v][j].y * a.scale) *
-                                   (ut[128 + (P >> 7)] * ut[P & 127]);
-            __builtin_nontemporal_store(z.x, o + P);
-            __builtin_nontemporal_store(z.y, o + P + L);
-        }
-    }
-}
-
 template <int SB> struct CombineArgs {
     int n, S, batch, nprod, ka, kb, wa, wb, ca;
     const cplx<float>* scratch;

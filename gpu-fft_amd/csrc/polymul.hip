@@ -2,8 +2,9 @@
 // two GPU_FFNT calls and a caller-side rounding for the same product,
 // example/test_ffnt_gpu_R_R.cu:137-162).
 //
-// A plan owns its root tables (generated on the GPU in FP64 in the
-// reference's FFNT layouts) and the scratch buffer of the split kernels.
+// A plan owns its root tables (generated on the GPU in FP64: the merged roots
+// of product.hpp, or the reference's FFNT layouts for the FP32 split) and the
+// scratch buffer of the split kernels.
 //   GPUFFT_PREC_F64        double in, double out (unrounded, like GPU_FFNT)
 //   GPUFFT_PREC_F32_SPLIT  int32 in, int64 out: the operands are split into
 //                          balanced base-2^w limbs, every limb product runs in
@@ -16,6 +17,7 @@
 #include <string>
 
 #include "fused.hpp"
+#include "product_launch.hpp"
 #include "status.hpp"
 
 using namespace gfa;
@@ -30,10 +32,10 @@ struct gpufft_polymul_plan_s {
     int ca;          // FP32 split: a split as a - 2^ca (0: none), plus the limb 2^ca J b
     void* jspec;     // FP32 split with ca: forward FFNT spectrum of J (complex float, L)
     int S, SB;       // sub-problem split
-    int rb;          // radix bits per LDS step of the product kernel
-    int e;           // log2 points per thread of the product kernel (2^(S-e) threads)
-    int cmb;         // FP64, SB > 0: 1 = top stages in the product kernel, 0 = separate pass (default)
-    void* root;      // forward FFNT root table (L entries)
+    int rb;          // FP32 split: radix bits per LDS step of the product kernel
+    int e;           // FP32 split: log2 points per thread of the product kernel (2^(S-e) threads)
+    int cmb;         // FP64, SB > 0: 1 = PHASE_TRANSFORM runs the combine too
+    void* root;      // FP64: merged roots (product.hpp); FP32 split: forward FFNT root table (L entries)
     void* iroot;
     void* twist;
     void* untwist;
@@ -41,7 +43,6 @@ struct gpufft_polymul_plan_s {
     void* wci;
     void* scratch;
     size_t scratch_bytes;
-    int* arrive;     // per-product arrival counters (max_batch), kept at 0 between launches
 };
 
 namespace {
@@ -49,11 +50,7 @@ namespace {
 constexpr int F64_MAX_S = 13;  // 2^13 doubles complex = 128 KiB of LDS
 constexpr int F32_MAX_S = 14;  // 2^14 floats complex = 128 KiB of LDS
 constexpr int MAX_SB = 3;
-#ifndef GFA_E64
-#define GFA_E64 4
-#endif
-
-
+constexpr int F64_E = 4;   // FP64 plans: log2 points per thread
 
 template <typename T> using ProdKernel = void (*)(ProdArgs<T>);
 
@@ -71,12 +68,6 @@ __global__ void fill_ones(float* p, long long n)
     if (i < n) p[i] = 1.0f;
 }
 
-__global__ void zero_ints(int* p, int n)
-{
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < n) p[i] = 0;
-}
-
 // Whether the product kernel exists for a sub-problem of 2^S points, 2^E
 // points per thread and radix-2^RB steps: the thread's groups of V loaded
 // positions must hold the 2^(S mod RB) partners of the register top step.
@@ -87,104 +78,92 @@ template <typename T, int S, int E, int PL, int RB> constexpr bool prod_ok()
     return RB <= E && S > E && ((1 << E) / V) / (1 << HB) >= 1;
 }
 
-// 2^E points per thread: 2^(S-E) threads per workgroup
-template <typename T, int PL, int RB, int E> ProdKernel<T> prod_kernel_rb(int S, int SB, int cmb)
+// FP32 split, 2^E points per thread: 2^(S-E) threads per workgroup
+template <int RB, int E> ProdKernel<float> prod_kernel_rb(int S, int SB)
 {
-    constexpr int SMAX = sizeof(T) == 8 ? F64_MAX_S : F32_MAX_S;
-    if constexpr (sizeof(T) == 8 && PL == PL_FOLD) {
-        if (cmb && S == SMAX) {
-            if (SB == 1) return &product_sub_kernel<T, SMAX, 1, E, PL, RB, true>;
-            if (SB == 2) return &product_sub_kernel<T, SMAX, 2, E, PL, RB, true>;
-            if (SB == 3) return &product_sub_kernel<T, SMAX, 3, E, PL, RB, true>;
-        }
-    }
 #define GFA_PK(SS, BB)                                                 \
-    if constexpr (prod_ok<T, SS, E, PL, RB>())                         \
-        if (S == SS && SB == BB) return &product_sub_kernel<T, SS, BB, E, PL, RB>;
-    if (SB > 0) {
-        GFA_PK(SMAX, 1)
-        GFA_PK(SMAX, 2)
-        GFA_PK(SMAX, 3)
-    } else {
-        GFA_PK(6, 0)
-        GFA_PK(7, 0)
-        GFA_PK(8, 0)
-        GFA_PK(9, 0)
-        GFA_PK(10, 0)
-        GFA_PK(11, 0)
-        GFA_PK(12, 0)
-        GFA_PK(13, 0)
-        if constexpr (SMAX >= 14) {
-            GFA_PK(14, 0)
-        }
-    }
+    if constexpr (prod_ok<float, SS, E, PL_FOLD_LIMB, RB>())           \
+        if (S == SS && SB == BB) return &product_sub_kernel<float, SS, BB, E, PL_FOLD_LIMB, RB>;
+    GFA_PK(7, 0)
+    GFA_PK(8, 0)
+    GFA_PK(9, 0)
+    GFA_PK(10, 0)
+    GFA_PK(11, 0)
+    GFA_PK(12, 0)
+    GFA_PK(13, 0)
+    GFA_PK(14, 0)
+    GFA_PK(14, 1)
+    GFA_PK(14, 2)
+    GFA_PK(14, 3)
 #undef GFA_PK
     return nullptr;
 }
 
-// radix bits per LDS step: 3 or 4 (double), 3..5 (float); points per thread
-// 2^e: 16 (double), 32 or 16 (float); both chosen per plan
-template <typename T, int PL, int E> ProdKernel<T> prod_kernel_e(int S, int SB, int rb, int cmb)
+// radix bits per LDS step 3..5, points per thread 2^e: 32 or 16; both chosen
+// per plan
+template <int E> ProdKernel<float> prod_kernel_e(int S, int SB, int rb)
 {
     switch (rb) {
-        case 3: return prod_kernel_rb<T, PL, 3, E>(S, SB, cmb);
-        case 4: return prod_kernel_rb<T, PL, 4, E>(S, SB, cmb);
+        case 3: return prod_kernel_rb<3, E>(S, SB);
+        case 4: return prod_kernel_rb<4, E>(S, SB);
         case 5:
-            if constexpr (sizeof(T) == 4 && E >= 5) return prod_kernel_rb<T, PL, 5, E>(S, SB, cmb);
+            if constexpr (E >= 5) return prod_kernel_rb<5, E>(S, SB);
             return nullptr;
         default: return nullptr;
     }
 }
 
-template <typename T, int PL> ProdKernel<T> prod_kernel(int S, int SB, int rb, int cmb, int e)
+ProdKernel<float> prod_kernel(int S, int SB, int rb, int e)
 {
-    if constexpr (sizeof(T) == 8) {
-        return e == GFA_E64 ? prod_kernel_e<T, PL, GFA_E64>(S, SB, rb, cmb) : nullptr;
-    } else {
-        if (e == 5) return prod_kernel_e<T, PL, 5>(S, SB, rb, cmb);
-        if (e == 4) return prod_kernel_e<T, PL, 4>(S, SB, rb, cmb);
-        return nullptr;
-    }
+    if (e == 5) return prod_kernel_e<5>(S, SB, rb);
+    if (e == 4) return prod_kernel_e<4>(S, SB, rb);
+    return nullptr;
 }
 
-template <typename T> int make_tables(gpufft_polymul_plan_s* pl, hipStream_t st)
+int make_f64_table(gpufft_polymul_plan_s* pl, hipStream_t st)
 {
-    size_t bytes = sizeof(cplx<T>) << pl->n;
+    hipError_t e = hipMalloc(&pl->root, sizeof(cplx<double>) * product_table_entries(pl->n, pl->SB));
+    if (e != hipSuccess) return fail_hip(e, "gpufft_polymul_plan_create: hipMalloc");
+    return launch_product_table(pl->root, pl->n, pl->SB, st, "gpufft_polymul_plan_create");
+}
+
+int make_f32_tables(gpufft_polymul_plan_s* pl, hipStream_t st)
+{
+    size_t bytes = sizeof(cplx<float>) << pl->n;
     void** dst[4] = {&pl->root, &pl->iroot, &pl->twist, &pl->untwist};
     for (void** d : dst) {
         hipError_t e = hipMalloc(d, bytes);
         if (e != hipSuccess) return fail_hip(e, "gpufft_polymul_plan_create: hipMalloc");
     }
     for (void** d : {&pl->wc, &pl->wci}) {
-        hipError_t e = hipMalloc(d, sizeof(cplx<T>) * 32);
+        hipError_t e = hipMalloc(d, sizeof(cplx<float>) * 32);
         if (e != hipSuccess) return fail_hip(e, "gpufft_polymul_plan_create: hipMalloc");
     }
-    int (*gen)(void*, int, int, int, void*) =
-        sizeof(T) == 8 ? gpufft_generate_table_f64 : gpufft_generate_table_f32;
     int s;
-    if ((s = gen(pl->root, GPUFFT_TABLE_FFNT_ROOT, pl->n, 0, st))) return s;
-    if ((s = gen(pl->iroot, GPUFFT_TABLE_FFNT_ROOT, pl->n, 1, st))) return s;
-    if ((s = gen(pl->twist, GPUFFT_TABLE_FFNT_TWIST, pl->n, 0, st))) return s;
-    if ((s = gen(pl->untwist, GPUFFT_TABLE_FFNT_TWIST, pl->n, 1, st))) return s;
-    if ((s = gen(pl->wc, GPUFFT_TABLE_STAGE_ROOTS, 5, 0, st))) return s;
-    if ((s = gen(pl->wci, GPUFFT_TABLE_STAGE_ROOTS, 5, 1, st))) return s;
+    if ((s = gpufft_generate_table_f32(pl->root, GPUFFT_TABLE_FFNT_ROOT, pl->n, 0, st))) return s;
+    if ((s = gpufft_generate_table_f32(pl->iroot, GPUFFT_TABLE_FFNT_ROOT, pl->n, 1, st))) return s;
+    if ((s = gpufft_generate_table_f32(pl->twist, GPUFFT_TABLE_FFNT_TWIST, pl->n, 0, st))) return s;
+    if ((s = gpufft_generate_table_f32(pl->untwist, GPUFFT_TABLE_FFNT_TWIST, pl->n, 1, st))) return s;
+    if ((s = gpufft_generate_table_f32(pl->wc, GPUFFT_TABLE_STAGE_ROOTS, 5, 0, st))) return s;
+    if ((s = gpufft_generate_table_f32(pl->wci, GPUFFT_TABLE_STAGE_ROOTS, 5, 1, st))) return s;
     return GPUFFT_OK;
 }
 
 void release(gpufft_polymul_plan_s* pl)
 {
     if (!pl) return;
-    void* ptrs[9] = {pl->root, pl->iroot, pl->twist, pl->untwist, pl->wc, pl->wci, pl->scratch,
-                     pl->arrive, pl->jspec};
+    void* ptrs[8] = {pl->root, pl->iroot, pl->twist, pl->untwist, pl->wc, pl->wci, pl->scratch,
+                     pl->jspec};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     delete pl;
 }
 
-template <typename T, int PL>
-int launch_products(const gpufft_polymul_plan_s* pl, const void* a, const void* b, T* out_direct,
-                    int batch, int cmb, hipStream_t st, const char* who)
+// FP32-split transforms and limb products into the plan's scratch
+int launch_split(const gpufft_polymul_plan_s* pl, const int32_t* a, const int32_t* b, int batch,
+                 hipStream_t st, const char* who)
 {
+    using T = float;
     ProdArgs<T> pa{};
     pa.n = pl->n;
     pa.S = pl->S;
@@ -200,9 +179,6 @@ int launch_products(const gpufft_polymul_plan_s* pl, const void* a, const void* 
     pa.b = b;
     pa.in_stride = 2LL << pl->n;
     pa.scratch = (cplx<T>*)pl->scratch;
-    pa.out = out_direct;
-    pa.out_stride = 2LL << pl->n;
-    pa.scale = mk<T>((T)(1.0 / (double)(1LL << pl->n)), (T)0);
     pa.wa = pl->wa;
     pa.ka = pl->ka;
     pa.ca = pl->ca;
@@ -216,8 +192,7 @@ int launch_products(const gpufft_polymul_plan_s* pl, const void* a, const void* 
     };
     pa.oa = pl->ka > 1 ? offset(pl->wa, pl->ka) : 0;
     pa.ob = pl->kb > 1 ? offset(pl->wb, pl->kb) : 0;
-    pa.arrive = pl->arrive;
-    ProdKernel<T> k = prod_kernel<T, PL>(pl->S, pl->SB, pl->rb, cmb, pl->e);
+    ProdKernel<T> k = prod_kernel(pl->S, pl->SB, pl->rb, pl->e);
     if (!k) return fail(GPUFFT_ERR_UNSUPPORTED, std::string(who) + ": no kernel for this size");
     const int threads = (1 << pl->S) >> pl->e;
     const long long groups = ((long long)batch + 7) / 8;
@@ -242,51 +217,33 @@ int run_f64(const gpufft_polymul_plan_s* plan, const double* a, const double* b,
             int batch, int phases, hipStream_t st, const char* who)
 {
     const long long N = 2LL << plan->n;
+    const int S = plan->S, SB = plan->SB;
+    const bool transform = phases & GPUFFT_PHASE_TRANSFORM;
+    // combine_in_kernel: PHASE_TRANSFORM writes the output, PHASE_COMBINE
+    // alone does nothing
+    const bool combine = SB > 0 && (plan->cmb ? transform : (phases & GPUFFT_PHASE_COMBINE) != 0);
     for (int b0 = 0; b0 < batch; b0 += plan->max_batch) {
         const int nb = std::min(plan->max_batch, batch - b0);
-        const double* pa = a + b0 * N;
-        const double* pb = b + b0 * N;
-        double* po = out + b0 * N;
-        // in-kernel combine: one launch does both phases (PHASE_TRANSFORM
-        // runs it, PHASE_COMBINE alone does nothing)
-        const int cmb = plan->cmb && plan->SB > 0;
-        if (phases & GPUFFT_PHASE_TRANSFORM)
-            if (int s = launch_products<double, PL_FOLD>(plan, pa, pb, po, nb, cmb, st, who)) return s;
-        if (plan->SB > 0 && !cmb && (phases & GPUFFT_PHASE_COMBINE)) {
-            // top SB inverse stages + scale + untwist + unfold
-            F64CombineArgs ca{};
-            ca.n = plan->n;
-            ca.S = plan->S;
-            ca.batch = nb;
-            ca.scratch = (const cplx<double>*)plan->scratch;
-            ca.itab = (const cplx<double>*)plan->iroot;
-            ca.untwist = (const cplx<double>*)plan->untwist;
-            ca.scale = 1.0 / (double)(1LL << plan->n);
-            ca.out = po;
-            ca.out_stride = N;
-            // 512 columns per workgroup, every workgroup inside one product
-            if (plan->S < 9) return fail(GPUFFT_ERR_UNSUPPORTED, std::string(who) + ": tile too small");
-            const unsigned blocks = (unsigned)((long long)nb << (plan->S - 9));
-            switch (plan->SB) {
-                case 1: hipLaunchKernelGGL(f64_combine_kernel<1>, dim3(blocks), dim3(256), 0, st, ca); break;
-                case 2: hipLaunchKernelGGL(f64_combine_kernel<2>, dim3(blocks), dim3(256), 0, st, ca); break;
-                case 3: hipLaunchKernelGGL(f64_combine_kernel<3>, dim3(blocks), dim3(256), 0, st, ca); break;
-                default: return fail(GPUFFT_ERR_UNSUPPORTED, std::string(who) + ": split too deep");
-            }
-            GFA_CHECK_LAUNCH(who);
-        }
+        if (transform)
+            if (int s = launch_product_f64(plan->n, S, SB, nb, plan->root, a + b0 * N, b + b0 * N,
+                                           out + b0 * N, plan->scratch, st, who))
+                return s;
+        if (combine)
+            if (int s = launch_combine_f64(plan->n, S, SB, nb, plan->root, plan->scratch, out + b0 * N,
+                                           st, who))
+                return s;
     }
     return ok();
 }
 
 // ---- products without allocation ----
-// Static device scratch of gpufft_polymul_f64_noalloc: the stage root
-// constants (64 complex doubles in the first 1 KiB, written by every call)
-// and the sub-problem results of products split over several workgroups.
+// Static device scratch of gpufft_polymul_f64_noalloc: the merged root table
+// (written by every call) and the sub-problem results of products split over
+// several workgroups, room for 64 MiB of them beside the largest table.
 // Each device holds its own copy from module load until the process ends;
 // calls that overlap in time on one device share it and race.
-constexpr size_t NOALLOC_BYTES = (size_t)64 << 20;
-constexpr size_t NOALLOC_CONST_BYTES = 1024;
+constexpr size_t NOALLOC_TABLE_BYTES = ((size_t)1 << 20) + 1024;  // n = 16, SB = 3: 2^16 + 64 entries
+constexpr size_t NOALLOC_BYTES = NOALLOC_TABLE_BYTES + ((size_t)64 << 20);
 static __device__ __align__(256) unsigned char scratch[NOALLOC_BYTES];
 
 constexpr int NOALLOC_MAX_DEVICES = 64;
@@ -364,10 +321,10 @@ int gpufft_polymul_plan_create(gpufft_polymul_plan* out, int ring_power, int pre
     // FP32: 16 points per thread (1024 threads) for full tiles of products
     // in one or two sub-problems; with more, the top-row gather's partner
     // loads spill at 128 VGPRs and 32 points per thread (256 VGPRs) is faster
-    pl->e = precision == GPUFFT_PREC_F64 ? GFA_E64 : (pl->S == F32_MAX_S && pl->SB <= 1 ? 4 : 5);
-    pl->cmb = 0;  // separate pass: measured faster at N = 2^16, batch 256
+    pl->e = precision == GPUFFT_PREC_F64 ? F64_E : (pl->S == F32_MAX_S && pl->SB <= 1 ? 4 : 5);
+    pl->cmb = 0;
     hipStream_t st = (hipStream_t)stream;
-    int s = precision == GPUFFT_PREC_F64 ? make_tables<double>(pl, st) : make_tables<float>(pl, st);
+    int s = precision == GPUFFT_PREC_F64 ? make_f64_table(pl, st) : make_f32_tables(pl, st);
     if (s) {
         release(pl);
         return s;
@@ -384,16 +341,7 @@ int gpufft_polymul_plan_create(gpufft_polymul_plan* out, int ring_power, int pre
             return fail_hip(e, "gpufft_polymul_plan_create: hipMalloc scratch");
         }
     }
-    if (precision == GPUFFT_PREC_F64 && pl->SB > 0) {
-        hipError_t e = hipMalloc((void**)&pl->arrive, sizeof(int) * (size_t)max_batch);
-        if (e != hipSuccess) {
-            release(pl);
-            return fail_hip(e, "gpufft_polymul_plan_create: hipMalloc counters");
-        }
-        hipLaunchKernelGGL(zero_ints, dim3((unsigned)((max_batch + 255) / 256)), dim3(256), 0, st,
-                           pl->arrive, max_batch);
-    }
-    // tables and counters are ready before the plan is used on any stream
+    // tables are ready before the plan is used on any stream
     hipError_t e = hipStreamSynchronize(st);
     if (e != hipSuccess) {
         release(pl);
@@ -447,8 +395,7 @@ int gpufft_polymul_i32_phases(gpufft_polymul_plan plan, const int32_t* a, const 
     for (int b0 = 0; b0 < batch; b0 += plan->max_batch) {
         const int nb = std::min(plan->max_batch, batch - b0);
         if (phases & GPUFFT_PHASE_TRANSFORM)
-            if (int s = launch_products<float, PL_FOLD_LIMB>(plan, a + b0 * N, b + b0 * N, nullptr,
-                                                             nb, 0, st, who))
+            if (int s = launch_split(plan, a + b0 * N, b + b0 * N, nb, st, who))
                 return s;
         if (!(phases & GPUFFT_PHASE_COMBINE)) continue;
         const long long nthreads_total = (long long)nb << plan->S;
@@ -503,7 +450,7 @@ int gpufft_polymul_plan_set_radix_bits(gpufft_polymul_plan plan, int radix_bits)
     if (radix_bits < 3 || radix_bits > hi)
         return fail(GPUFFT_ERR_INVALID_ARGUMENT, std::string(who) + ": radix_bits out of range");
     if (plan->precision == GPUFFT_PREC_F32_SPLIT &&
-        !prod_kernel<float, PL_FOLD_LIMB>(plan->S, plan->SB, radix_bits, 0, plan->e))
+        !prod_kernel(plan->S, plan->SB, radix_bits, plan->e))
         return fail(GPUFFT_ERR_UNSUPPORTED,
                     std::string(who) + ": no kernel for this radix at the plan's points per thread");
     plan->rb = radix_bits;
@@ -514,11 +461,11 @@ int gpufft_polymul_plan_set_thread_points(gpufft_polymul_plan plan, int log2_poi
 {
     const char* who = "gpufft_polymul_plan_set_thread_points";
     if (!plan) return fail(GPUFFT_ERR_NULL_POINTER, std::string(who) + ": plan is NULL");
-    const bool okv = plan->precision == GPUFFT_PREC_F64 ? log2_points == GFA_E64
+    const bool okv = plan->precision == GPUFFT_PREC_F64 ? log2_points == F64_E
                                                         : (log2_points == 4 || log2_points == 5);
     if (!okv) return fail(GPUFFT_ERR_INVALID_ARGUMENT, std::string(who) + ": unsupported points per thread");
-    if (!prod_kernel<float, PL_FOLD_LIMB>(plan->S, plan->SB, plan->rb, 0, log2_points) &&
-        plan->precision == GPUFFT_PREC_F32_SPLIT)
+    if (plan->precision == GPUFFT_PREC_F32_SPLIT &&
+        !prod_kernel(plan->S, plan->SB, plan->rb, log2_points))
         return fail(GPUFFT_ERR_UNSUPPORTED, std::string(who) + ": no kernel for this size and radix");
     plan->e = log2_points;
     return ok();
@@ -616,27 +563,17 @@ int gpufft_polymul_f64_noalloc(const double* a, const double* b, double* out, in
     pl.ka = pl.kb = 1;
     pl.S = std::min(n, F64_MAX_S);
     pl.SB = n - pl.S;
-    pl.rb = 4;
-    pl.e = GFA_E64;
-    pl.cmb = 0;
-    pl.root = const_cast<void*>(root_table);
-    pl.iroot = const_cast<void*>(inv_root_table);
-    pl.twist = const_cast<void*>(twist);
-    pl.untwist = const_cast<void*>(untwist);
-    cplx<double>* consts = (cplx<double>*)base;
-    pl.wc = consts;
-    pl.wci = consts + 32;
+    pl.root = base;
     // the sub-problem results of one launch must fit the rest of the array:
     // the batch runs in launches of at most that many products
     const size_t per_product = pl.SB > 0 ? (sizeof(cplx<double>) << n) : 0;
-    const size_t room = NOALLOC_BYTES - NOALLOC_CONST_BYTES;
+    const size_t room = NOALLOC_BYTES - NOALLOC_TABLE_BYTES;
     pl.max_batch = per_product ? (int)std::min<size_t>(room / per_product, (size_t)batch) : batch;
-    pl.scratch = pl.SB > 0 ? (void*)((unsigned char*)base + NOALLOC_CONST_BYTES) : nullptr;
+    pl.scratch = pl.SB > 0 ? (void*)((unsigned char*)base + NOALLOC_TABLE_BYTES) : nullptr;
     pl.scratch_bytes = pl.SB > 0 ? room : 0;
-    // stage root constants: rewritten by every call (a kernel, so the call
-    // can be captured into a graph), ahead of the product kernels on `st`
-    if (int s = gpufft_generate_table_f64(pl.wc, GPUFFT_TABLE_STAGE_ROOTS, 5, 0, st)) return s;
-    if (int s = gpufft_generate_table_f64(pl.wci, GPUFFT_TABLE_STAGE_ROOTS, 5, 1, st)) return s;
+    // the merged roots: rewritten by every call (a kernel, so the call can be
+    // captured into a graph), ahead of the product kernels on `st`
+    if (int s = launch_product_table(pl.root, n, pl.SB, st, who)) return s;
     return run_f64(&pl, a, b, out, batch, GPUFFT_PHASE_ALL, st, who);
 }
 

@@ -1,0 +1,20 @@
+// Launches of the fused FP64 product kernels (product.hip).
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+namespace gfa {
+
+// Entries of the merged root table: 2^n roots, 4^SB residue powers.
+inline size_t product_table_entries(int n, int SB) { return ((size_t)1 << n) + ((size_t)1 << (2 * SB)); }
+
+int launch_product_table(void* w, int n, int SB, hipStream_t st, const char* who);
+// Products of 2^n complex points in 2^SB sub-problems of 2^S: into out
+// (SB = 0) or the sub-results in scratch.
+int launch_product_f64(int n, int S, int SB, int batch, const void* w, const double* a, const double* b,
+                       double* out, void* scratch, hipStream_t st, const char* who);
+// The top SB inverse stages from scratch to out.
+int launch_combine_f64(int n, int S, int SB, int batch, const void* w, const void* scratch, double* out,
+                       hipStream_t st, const char* who);
+
+}  // namespace gfa

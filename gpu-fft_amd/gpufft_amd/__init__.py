@@ -281,9 +281,9 @@ class PolymulPlan:
 
     @property
     def thread_points(self):
-        """log2 of the points per thread of the product kernel: 4 for FP64
-        (512 threads per 2^13-point sub-problem); 5 or 4 for the FP32 split
-        (512 or 1024 threads per 2^14-point sub-problem)."""
+        """log2 of the points per thread of the product kernel: 4 for FP64;
+        5 or 4 for the FP32 split (512 or 1024 threads per 2^14-point
+        sub-problem)."""
         return _lib.gpufft_polymul_plan_get_thread_points(self.handle)
 
     @thread_points.setter
@@ -292,8 +292,8 @@ class PolymulPlan:
 
     @property
     def combine_in_kernel(self):
-        """FP64 plans of ring_power >= 15: last inverse stages in the product
-        kernel (True) or in a second launch (False, default)."""
+        """FP64 plans of ring_power >= 15: the launch of the last inverse stages
+        belongs to PHASE_TRANSFORM (True) or PHASE_COMBINE (False, default)."""
         return bool(_lib.gpufft_polymul_plan_get_combine(self.handle))
 
     @combine_in_kernel.setter

@@ -189,14 +189,13 @@ int gpufft_polymul_plan_create(gpufft_polymul_plan* out, int ring_power, int pre
                                int b_limbs, void* stream);
 int gpufft_polymul_plan_destroy(gpufft_polymul_plan plan);
 size_t gpufft_polymul_plan_scratch_bytes(gpufft_polymul_plan plan);
-/* Radix of the LDS steps of the product kernel, 2^radix_bits: 3 or 4 for
- * GPUFFT_PREC_F64, 3..5 for GPUFFT_PREC_F32_SPLIT (default 4).  Results do
- * not depend on it beyond rounding; the autotuner (gpufft_amd.autotune)
- * sets it per ring size and device. */
+/* Radix of the LDS steps of the product kernel, 2^radix_bits: 3..5 for
+ * GPUFFT_PREC_F32_SPLIT (default 4).  Results do not depend on it beyond
+ * rounding.  GPUFFT_PREC_F64 plans accept 3 and 4 and run the same kernel. */
 int gpufft_polymul_plan_set_radix_bits(gpufft_polymul_plan plan, int radix_bits);
 int gpufft_polymul_plan_get_radix_bits(gpufft_polymul_plan plan);
 /* Points per thread of the product kernel, 2^log2_points: 4 for
- * GPUFFT_PREC_F64 (512 threads per 2^13-point sub-problem); 5 (512
+ * GPUFFT_PREC_F64; 5 (512
  * threads) or 4 (1024 threads) per 2^14-point sub-problem for
  * GPUFFT_PREC_F32_SPLIT (default 4 for ring_power 15 and 16, 5 otherwise).
  * Results do not depend on it beyond rounding.
@@ -205,12 +204,11 @@ int gpufft_polymul_plan_get_radix_bits(gpufft_polymul_plan plan);
 int gpufft_polymul_plan_set_thread_points(gpufft_polymul_plan plan, int log2_points);
 int gpufft_polymul_plan_get_thread_points(gpufft_polymul_plan plan);
 /* GPUFFT_PREC_F64 plans whose product spans several workgroups (ring_power
- * >= 15): in_kernel = 1 runs the last inverse stages inside the product
- * kernel, in the workgroup that finishes a product last (one launch); 0
- * (default) runs them as a second, streaming launch.  On MI355X the second
- * launch is faster: the in-kernel form's device-scope release/acquire write
- * back and invalidate L2, which the product kernel's input reads rely on.
- * Other plans ignore the setting (get returns 0).  Same results either way. */
+ * >= 15) run their last inverse stages as a second, streaming launch.
+ * in_kernel = 1 makes it part of GPUFFT_PHASE_TRANSFORM (which then writes
+ * the output, and GPUFFT_PHASE_COMBINE alone does nothing); 0 (default) of
+ * GPUFFT_PHASE_COMBINE.  Other plans ignore the setting (get returns 0).
+ * Same results either way. */
 int gpufft_polymul_plan_set_combine(gpufft_polymul_plan plan, int in_kernel);
 int gpufft_polymul_plan_get_combine(gpufft_polymul_plan plan);
 /* GPUFFT_PREC_F32_SPLIT plans: split a - 2^center_log2 instead of a (0, the
@@ -229,8 +227,8 @@ int gpufft_polymul_i32(gpufft_polymul_plan plan, const int32_t* a, const int32_t
  * schedule or time them apart: GPUFFT_PHASE_TRANSFORM runs the forward
  * transforms, products and inverse sub-transforms into the plan's scratch,
  * GPUFFT_PHASE_COMBINE the last inverse stages and the output (for plans
- * whose whole product fits one workgroup, and for FP64 plans with the
- * in-kernel combine, the first phase writes the output and the second does
+ * whose whole product fits one workgroup, and for FP64 plans with combine
+ * in_kernel set, the first phase writes the output and the second does
  * nothing).  A combine must follow the transform of the same inputs on the
  * same plan, with batch <= max_batch. */
 #define GPUFFT_PHASE_TRANSFORM 1
@@ -248,10 +246,11 @@ int gpufft_polymul_i32_phases(gpufft_polymul_plan plan, const int32_t* a, const 
  * harnesses that forbid hipMalloc).  The caller passes the inputs, the
  * output and the four FFNT tables of ring N = 2^ring_power (N/2 entries
  * each, the layouts GPU_FFNT takes: twist, untwist, root and inverse root,
- * e.g. from gpufft_generate_table_f64); the library uses a static device
- * array of 64 MiB (per device, held until the process ends) for the stage
- * constants and the sub-problem results, so the batch runs in launches of
- * at most 63 MiB / (8 N) products for ring_power >= 15.  ring_power 7..17
+ * e.g. from gpufft_generate_table_f64; the kernels take their roots from a
+ * table that the call generates, so these are only checked for NULL); the
+ * library uses a static device array of 65 MiB (per device, held until the
+ * process ends) for that table and the sub-problem results, so the batch
+ * runs in launches of at most 64 MiB / (8 N) products for ring_power >= 15.  ring_power 7..17
  * (else GPUFFT_ERR_INVALID_ARGUMENT); a, b, out: double [batch][N]; out is
  * the unrounded product mod X^N+1, equal to gpufft_polymul_f64's.  Calls
  * that overlap in time on one device share the array and race; calls on one
