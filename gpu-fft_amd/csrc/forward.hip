@@ -1,0 +1,23 @@
+// Launch of the one-launch double forward transforms (forward.hpp).
+#include "forward.hpp"
+
+#include <algorithm>
+
+#include "product_launch.hpp"
+
+namespace gfa {
+
+void launch_forward13(const OneArgs<double>& a, int SB, bool fold, hipStream_t st)
+{
+    using Fn = void (*)(OneArgs<double>);
+    static constexpr Fn fn[2][3] = {
+        {&forward13_kernel<1, false>, &forward13_kernel<2, false>, &forward13_kernel<3, false>},
+        {&forward13_kernel<1, true>, &forward13_kernel<2, true>, &forward13_kernel<3, true>}};
+    // 8 transforms at a time, one per XCD, 2^SB workgroups each
+    const long long unit = 8LL << SB;
+    const long long items = (((long long)a.batch + 7) / 8 * 8) << SB;
+    const int grid = (int)std::max<long long>(unit, persistent_grid(items, 1) / unit * unit);
+    hipLaunchKernelGGL(fn[fold][SB - 1], dim3((unsigned)grid), dim3(512), 0, st, a);
+}
+
+}  // namespace gfa

@@ -20,7 +20,7 @@ struct Launch {
 
 template <int S, int SB> Launch shape_of()
 {
-    using P = ProductShape<S>;
+    using P = SubShape<S>;
     return {&product_kernel<S, SB, false>, &product_kernel<S, SB, true>, P::NT, P::PER, P::RESIDENT};
 }
 
@@ -45,17 +45,6 @@ Launch select(int S, int SB)
             }
         default: return {};
     }
-}
-
-// Workgroups of a persistent launch: what the CUs hold at once, if there is
-// as much work.
-int grid_of(long long items, int resident)
-{
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 8)
-        cus = 256;
-    return (int)std::min<long long>(items, (long long)cus * resident);
 }
 
 }  // namespace
@@ -84,7 +73,7 @@ int launch_product_f64(int n, int S, int SB, int batch, const void* w, const dou
     // split products: 8 at a time, one per XCD, 2^SB workgroups each
     const long long unit = SB > 0 ? 8LL << SB : 1;
     const long long items = SB > 0 ? (((long long)batch + 7) / 8 * 8) << SB : ((long long)batch + l.per - 1) / l.per;
-    const int grid = (int)std::max<long long>(unit, grid_of(items, l.resident) / unit * unit);
+    const int grid = (int)std::max<long long>(unit, persistent_grid(items, l.resident) / unit * unit);
     hipLaunchKernelGGL(grid == items ? l.once : l.k, dim3((unsigned)grid), dim3(l.threads), 0, st, pa);
     GFA_CHECK_LAUNCH(who);
     return GPUFFT_OK;

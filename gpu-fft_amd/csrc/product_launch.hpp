@@ -3,10 +3,23 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 namespace gfa {
 
 // Entries of the merged root table: 2^n roots, 4^SB residue powers.
 inline size_t product_table_entries(int n, int SB) { return ((size_t)1 << n) + ((size_t)1 << (2 * SB)); }
+
+// Workgroups of a persistent launch of which `resident` share a CU: what the
+// CUs hold at once, if there is as much work.
+inline int persistent_grid(long long items, int resident)
+{
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 64)
+        cus = 256;
+    return (int)std::min<long long>(items, (long long)cus * resident);
+}
 
 int launch_product_table(void* w, int n, int SB, hipStream_t st, const char* who);
 // Products of 2^n complex points in 2^SB sub-problems of 2^S: into out

@@ -122,6 +122,8 @@ int run_transform(int mode, int n, int batch, int nega, const cplx<T>* tab,
     return ok();
 }
 
+void launch_forward13(const OneArgs<double>& a, int SB, bool fold, hipStream_t st);  // forward.hip
+
 // Out-of-place calls (R_R, FFNT) of 2^n points, n = S + SB with S the LDS
 // tile (13 double, 14 float) and SB = 1..3 (oneshot.hpp): the forward is one
 // launch of Q = 2^SB workgroups per transform; the inverse is a launch of
@@ -139,7 +141,6 @@ template <> struct OneCfg<double> {
 };
 template <> struct OneCfg<float> {
     static constexpr int S = 14, E = 5, RB = 4;   // forward: 512 threads, 32 points each
-    static constexpr int SI = 13, EI = 5;         // inverse: 256 threads, 32 points each
 };
 
 template <typename T> using OneFn = void (*)(OneArgs<T>);
@@ -149,7 +150,9 @@ template <typename T, int SB> OneFn<T> select_forward_sb(int lk)
 {
     constexpr int S = OneCfg<T>::S, E = OneCfg<T>::E, RB = OneCfg<T>::RB;
     if (lk == LD_REAL) return &fwd_sub_kernel<T, S, SB, E, RB, PL_REAL>;
-    if (lk == LD_FOLD) return &fwd_sub_kernel<T, S, SB, E, RB, PL_FOLD>;
+    if constexpr (sizeof(T) == 8 || SB < 3) {  // the rest: prefer_passes
+        if (lk == LD_FOLD) return &fwd_sub_kernel<T, S, SB, E, RB, PL_FOLD>;
+    }
     return nullptr;
 }
 
@@ -158,6 +161,32 @@ template <typename T, int SB> TopFn<T> select_top_sb(int sk)  // SB = 2..4
     if (sk == ST_REAL) return &inv_top_kernel<T, SB, ST_REAL>;
     if (sk == ST_UNFOLD) return &inv_top_kernel<T, SB, ST_UNFOLD>;
     return nullptr;
+}
+
+// Where the pass chain is faster than this path (us, both sides measured, chain
+// against this path):
+//   FP64 forward: few transforms (the chain's workgroups are smaller): FFNT of
+//     2^16 points x 2: 12.4 / 17.5, x 8 17.0 / 17.8, x 16 21.1 / 18.1; of 2^15
+//     x 2 11.6 / 12.3, x 8 13.6 / 12.7; R_R of 2^16 x 2 11.6 / 12.5, x 8 15.8 /
+//     12.8.  FFNT of 2^16 points has 8 workgroups to a transform: past 32
+//     transforms a second, emptier wave: x 36 32.8 / 40.5, x 64 43.3 / 43.8,
+//     x 128 85 / 74.
+//   FP32 inverse: R_R 2^15 x 128 17.3 / 20.7, x 1024 92 / 108; FFNT 2^15 points
+//     x 256 52 / 61, x 1 10.5 / 14.0, 2^16 x 1 10.7 / 14.9.
+//   FP32 forward up to 2^20 points in the launch (FFNT 2^15 x 16: 11.3 / 14.8, x
+//     32 14.1 / 14.9, x 64 19.1 / 15.1; R_R 2^16 x 16 13.4 / 13.6, x 32 20 / 13.6;
+//     R_R 2^15 x 16 10.5 / 12.4, x 32 13.3 / 12.6), and FFNT of 2^17 points (x 2
+//     10.7 / 22.5, x 64 51 / 60).
+template <typename T> bool prefer_passes(bool forward, int n, int batch, bool fold)
+{
+    const long long points = (long long)batch << n;
+    if constexpr (sizeof(T) == 8) {
+        if (!forward) return false;
+        if (n == 16) return batch <= (fold ? 8 : 2) || (fold && batch > 32 && batch <= 64);
+        return n == 15 && fold && batch <= 2;
+    }
+    if (!forward || (n == 17 && fold)) return true;
+    return points <= (n == 15 && !fold ? 1LL << 19 : 1LL << 20);
 }
 
 // Returns true and launches when this path covers the transform (status in
@@ -170,6 +199,7 @@ bool run_oneshot(int mode, int n, int batch, int nega, const cplx<T>* tab,
     constexpr int S = OneCfg<T>::S, E = OneCfg<T>::E, RB = OneCfg<T>::RB;
     const int SB = n - S;
     if (SB < 1 || SB > 3) return false;
+    if (prefer_passes<T>(mode == MODE_STD_FWD, n, batch, io.lk == LD_FOLD)) return false;
     OneArgs<T> a{};
     a.n = n;
     a.batch = batch;
@@ -185,39 +215,55 @@ bool run_oneshot(int mode, int n, int batch, int nega, const cplx<T>* tab,
     a.do_scale = io.do_scale ? 1 : 0;
     a.scale = io.do_scale ? io.scale : mk<T>(T(1), T(0));
     if (mode == MODE_STD_FWD && io.sk == ST_CPLX && (io.lk == LD_REAL || io.lk == LD_FOLD)) {
-        OneFn<T> fn = SB == 1 ? select_forward_sb<T, 1>(io.lk)
-                    : SB == 2 ? select_forward_sb<T, 2>(io.lk)
-                              : select_forward_sb<T, 3>(io.lk);
         const long long blocks = (((long long)batch + 7) / 8) * 8 * (1LL << SB);
         if (blocks > 0x7fffffffLL) {
             *status = fail(GPUFFT_ERR_INVALID_ARGUMENT, std::string(who) + ": batch too large");
             return true;
         }
-        hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3((1 << S) >> E), 0, stream, a);
-    } else if (mode == MODE_STD_INV && (io.lk == LD_CPLX || io.lk == LD_MUL) &&
-               (io.sk == ST_REAL || io.sk == ST_UNFOLD)) {
-        constexpr int SI = OneCfg<T>::SI, EI = OneCfg<T>::EI;
-        const int SBI = n - SI;  // 2..4
-        const long long blocks1 = (long long)batch << SBI;
-        static_assert(SI >= 9, "the second inverse launch takes 512 columns per workgroup");
-        const long long blocks2 = (long long)batch << (SI - 9);
-        if (blocks1 > 0x7fffffffLL || blocks2 > 0x7fffffffLL) {
-            *status = fail(GPUFFT_ERR_INVALID_ARGUMENT, std::string(who) + ": batch too large");
+        // FP64: the persistent form past one workgroup per CU (R_R 2^14 x
+        // 512: 34.7 us against 50.8, FFNT 2^15 points x 72 26.0 against 29.5, x
+        // 512 95 against 127); up to there its longer start counts (FFNT 2^15 x
+        // 32: 15.7 against 13.4, x 64 17.9 against 17.5)
+        bool launched = false;
+        if constexpr (sizeof(T) == 8) {
+            launched = blocks > 256;
+            if (launched) launch_forward13(a, SB, io.lk == LD_FOLD, stream);
+        }
+        if (!launched) {
+            OneFn<T> fn = SB == 1 ? select_forward_sb<T, 1>(io.lk)
+                        : SB == 2 ? select_forward_sb<T, 2>(io.lk)
+                                  : select_forward_sb<T, 3>(io.lk);
+            hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3((1 << S) >> E), 0, stream, a);
+        }
+        hipError_t e = hipGetLastError();
+        *status = e != hipSuccess ? fail_hip(e, who) : ok();
+        return true;
+    }
+    if constexpr (sizeof(T) == 8) {
+        if (mode == MODE_STD_INV && (io.lk == LD_CPLX || io.lk == LD_MUL) &&
+            (io.sk == ST_REAL || io.sk == ST_UNFOLD)) {
+            constexpr int SI = OneCfg<T>::SI, EI = OneCfg<T>::EI;
+            const int SBI = n - SI;  // 2..4
+            const long long blocks1 = (long long)batch << SBI;
+            static_assert(SI >= 9, "the second inverse launch takes 512 columns per workgroup");
+            const long long blocks2 = (long long)batch << (SI - 9);
+            if (blocks1 > 0x7fffffffLL || blocks2 > 0x7fffffffLL) {
+                *status = fail(GPUFFT_ERR_INVALID_ARGUMENT, std::string(who) + ": batch too large");
+                return true;
+            }
+            OneFn<T> f1 = io.lk == LD_MUL ? &inv_local_kernel<T, SI, EI, RB, LD_MUL>
+                                          : &inv_local_kernel<T, SI, EI, RB, LD_CPLX>;
+            hipLaunchKernelGGL(f1, dim3((unsigned)blocks1), dim3((1 << SI) >> EI), 0, stream, a);
+            TopFn<T> f2 = SBI == 2 ? select_top_sb<T, 2>(io.sk)
+                        : SBI == 3 ? select_top_sb<T, 3>(io.sk)
+                                   : select_top_sb<T, 4>(io.sk);
+            hipLaunchKernelGGL(f2, dim3((unsigned)blocks2), dim3(256), 0, stream, a, SI);
+            hipError_t e = hipGetLastError();
+            *status = e != hipSuccess ? fail_hip(e, who) : ok();
             return true;
         }
-        OneFn<T> f1 = io.lk == LD_MUL ? &inv_local_kernel<T, SI, EI, RB, LD_MUL>
-                                      : &inv_local_kernel<T, SI, EI, RB, LD_CPLX>;
-        hipLaunchKernelGGL(f1, dim3((unsigned)blocks1), dim3((1 << SI) >> EI), 0, stream, a);
-        TopFn<T> f2 = SBI == 2 ? select_top_sb<T, 2>(io.sk)
-                    : SBI == 3 ? select_top_sb<T, 3>(io.sk)
-                               : select_top_sb<T, 4>(io.sk);
-        hipLaunchKernelGGL(f2, dim3((unsigned)blocks2), dim3(256), 0, stream, a, SI);
-    } else {
-        return false;
     }
-    hipError_t e = hipGetLastError();
-    *status = e != hipSuccess ? fail_hip(e, who) : ok();
-    return true;
+    return false;
 }
 
 }  // namespace gfa
