@@ -1094,6 +1094,51 @@ __device__ __forceinline__ void dispatch_s(cplx<T>* lds, const BArgs& ba, const 
     }
 }
 
+// The workgroup's items: its home queue's, then the other queues'.  Which of
+// those still hold items is one read of all counters by the first wavefront: an
+// atomic on every queue by every workgroup, all on one cache line, took 11 us
+// at the end of a launch (3 products FP64 50 -> 39 us, 700 FP32 1006 -> 957).
+struct Puller {
+    int home;
+    bool open;  // the home queue may hold items
+
+    // Index of the next item, -1 once all queues are exhausted.
+    __device__ __forceinline__ int next(const BArgs& ba, int tid, int* sh_item)
+    {
+        if (tid < 64) {
+            int got = -1, x = home;
+            bool look = open;
+            for (;;) {
+                if (!look) {
+                    bool has = false;
+                    const int y = (home + tid) % NQ;
+                    if (tid < NQ)
+                        has = __hip_atomic_load(ba.next_item + y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <
+                              ba.qlen[y];
+                    const unsigned long long m = __ballot(has);
+                    if (m == 0) break;
+                    x = (home + __ffsll(m) - 1) % NQ;
+                }
+                look = false;
+                int it = 0;
+                if (tid == 0) it = atomicAdd(ba.next_item + x, 1);
+                it = __builtin_amdgcn_readfirstlane(it);
+                if (it < ba.qlen[x]) {  // else the queue is exhausted, and seen so from now on
+                    got = ba.qbeg[x] + it;
+                    break;
+                }
+            }
+            if (tid == 0) *sh_item = got < 0 ? -1 : got | (x == home ? 0 : 1 << 30);
+        }
+        __syncthreads();
+        const int s = __builtin_amdgcn_readfirstlane(*sh_item);
+        __syncthreads();
+        if (s < 0) return -1;
+        open = (s >> 30) == 0;
+        return s & ~(1 << 30);
+    }
+};
+
 // FP32: TILE = 14, one 128 KiB workgroup per CU; TILE = 13, 64 KiB
 // workgroups, compiled for 4 waves per SIMD so that two of them share a CU.
 // FP64: TILE = 13, one 128 KiB workgroup per CU.
@@ -1109,30 +1154,24 @@ void batched_kernel(BArgs ba)
     __shared__ int sh_item;
     __shared__ int sh_last;
     const int tid = threadIdx.x;
-    const int home = (int)(blockIdx.x % NQ);
-    for (int r = 0; r < NQ; r++) {
-        const int x = (home + r) % NQ;
-        for (;;) {
-            if (tid == 0) sh_item = atomicAdd(ba.next_item + x, 1);
-            __syncthreads();
-            const int it = sh_item;
-            __syncthreads();
-            if (it >= ba.qlen[x]) break;  // queue x is exhausted
-            // the item's records are read from memory, which the compiler
-            // cannot prove uniform: scalar copies keep the table resources in
-            // scalar registers (a buffer load through a resource in vector
-            // registers becomes a loop over lanes)
-            const int2 it2 = ba.items[ba.qbeg[x] + it];
-            const int2 item = make_int2(__builtin_amdgcn_readfirstlane(it2.x),
-                                        __builtin_amdgcn_readfirstlane(it2.y));
-            const BProd pr = uniform_copy(ba.prods[item.x]);
-            const BTables tb = uniform_copy(ba.tabs[pr.tabset]);
-            if (pr.kind == KIND_NEGA)
-                dispatch_s<T, KIND_NEGA, RB, TILE>(lds, ba, pr, tb, item.x, item.y, tid, &sh_last);
-            else
-                dispatch_s<T, KIND_LINEAR, RB, TILE>(lds, ba, pr, tb, item.x, item.y, tid, &sh_last);
-            __syncthreads();
-        }
+    Puller pull{(int)(blockIdx.x % NQ), true};
+    for (;;) {
+        const int it = pull.next(ba, tid, &sh_item);
+        if (it < 0) break;
+        // the item's records are read from memory, which the compiler
+        // cannot prove uniform: scalar copies keep the table resources in
+        // scalar registers (a buffer load through a resource in vector
+        // registers becomes a loop over lanes)
+        const int2 it2 = ba.items[it];
+        const int2 item = make_int2(__builtin_amdgcn_readfirstlane(it2.x),
+                                    __builtin_amdgcn_readfirstlane(it2.y));
+        const BProd pr = uniform_copy(ba.prods[item.x]);
+        const BTables tb = uniform_copy(ba.tabs[pr.tabset]);
+        if (pr.kind == KIND_NEGA)
+            dispatch_s<T, KIND_NEGA, RB, TILE>(lds, ba, pr, tb, item.x, item.y, tid, &sh_last);
+        else
+            dispatch_s<T, KIND_LINEAR, RB, TILE>(lds, ba, pr, tb, item.x, item.y, tid, &sh_last);
+        __syncthreads();
     }
     // The last workgroup to leave clears the queue, arrival and exit
     // counters for the next launch (every other workgroup has made its last
@@ -1142,7 +1181,8 @@ void batched_kernel(BArgs ba)
     __syncthreads();
     if (sh_last) {
         for (int i = tid; i < NQ; i += BT) atomicExch(ba.next_item + i, 0);
-        for (int i = tid; i < ba.count; i += BT) atomicExch(ba.arrive + i, 0);
+        if (ba.cmb)
+            for (int i = tid; i < ba.count; i += BT) atomicExch(ba.arrive + i, 0);
         if (tid == 0) atomicExch(ba.exited, 0);
     }
 }
