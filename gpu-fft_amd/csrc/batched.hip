@@ -1098,46 +1098,46 @@ __device__ __forceinline__ void dispatch_s(cplx<T>* lds, const BArgs& ba, const 
 // those still hold items is one read of all counters by the first wavefront: an
 // atomic on every queue by every workgroup, all on one cache line, took 11 us
 // at the end of a launch (3 products FP64 50 -> 39 us, 700 FP32 1006 -> 957).
-struct Puller {
-    int home;
-    bool open;  // the home queue may hold items
-
-    // Index of the next item, -1 once all queues are exhausted.
-    __device__ __forceinline__ int next(const BArgs& ba, int tid, int* sh_item)
-    {
-        if (tid < 64) {
-            int got = -1, x = home;
-            bool look = open;
-            for (;;) {
-                if (!look) {
-                    bool has = false;
-                    const int y = (home + tid) % NQ;
-                    if (tid < NQ)
-                        has = __hip_atomic_load(ba.next_item + y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <
-                              ba.qlen[y];
-                    const unsigned long long m = __ballot(has);
-                    if (m == 0) break;
-                    x = (home + __ffsll(m) - 1) % NQ;
-                }
-                look = false;
-                int it = 0;
-                if (tid == 0) it = atomicAdd(ba.next_item + x, 1);
-                it = __builtin_amdgcn_readfirstlane(it);
-                if (it < ba.qlen[x]) {  // else the queue is exhausted, and seen so from now on
-                    got = ba.qbeg[x] + it;
-                    break;
-                }
+// Index of the next item, -1 once all queues are exhausted.  sh: the index, and
+// whether the home queue is known to be exhausted (set to 0 by the first
+// wavefront before the first call; in LDS, as registers held across the items
+// cost the FP32 kernels spills: 4096 products on the smaller tile 4.81 -> 5.03 ms).
+__device__ __forceinline__ int next_item(const BArgs& ba, int tid, int* sh)
+{
+    if (tid < 64) {
+        const int home = (int)(blockIdx.x % NQ);
+        int got = -1, x = home;
+        bool look = sh[1] != 0;
+        for (;;) {
+            if (look) {
+                bool has = false;
+                const int y = (home + tid) % NQ;
+                if (tid < NQ)
+                    has = __hip_atomic_load(ba.next_item + y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <
+                          ba.qlen[y];
+                const unsigned long long m = __ballot(has);
+                if (m == 0) break;
+                x = (home + __ffsll(m) - 1) % NQ;
             }
-            if (tid == 0) *sh_item = got < 0 ? -1 : got | (x == home ? 0 : 1 << 30);
+            look = true;
+            int it = 0;
+            if (tid == 0) it = atomicAdd(ba.next_item + x, 1);
+            it = __builtin_amdgcn_readfirstlane(it);
+            if (it < ba.qlen[x]) {  // else the queue is exhausted, and seen so from now on
+                got = ba.qbeg[x] + it;
+                break;
+            }
         }
-        __syncthreads();
-        const int s = __builtin_amdgcn_readfirstlane(*sh_item);
-        __syncthreads();
-        if (s < 0) return -1;
-        open = (s >> 30) == 0;
-        return s & ~(1 << 30);
+        if (tid == 0) {
+            sh[0] = got;
+            sh[1] = x != home;
+        }
     }
-};
+    __syncthreads();
+    const int s = sh[0];
+    __syncthreads();
+    return s;
+}
 
 // FP32: TILE = 14, one 128 KiB workgroup per CU; TILE = 13, 64 KiB
 // workgroups, compiled for 4 waves per SIMD so that two of them share a CU.
@@ -1151,12 +1151,12 @@ void batched_kernel(BArgs ba)
     // split twist tables (at most 2^(TILE-7) + 128 entries)
     constexpr int EXTRA = sizeof(T) == 8 ? (1 << SBMAX) + (1 << (TILE - 7)) + 128 : 0;
     __shared__ cplx<T> lds[(1 << TILE) + EXTRA];
-    __shared__ int sh_item;
+    __shared__ int sh_item[2];
     __shared__ int sh_last;
     const int tid = threadIdx.x;
-    Puller pull{(int)(blockIdx.x % NQ), true};
+    if (tid == 0) sh_item[1] = 0;
     for (;;) {
-        const int it = pull.next(ba, tid, &sh_item);
+        const int it = next_item(ba, tid, sh_item);
         if (it < 0) break;
         // the item's records are read from memory, which the compiler
         // cannot prove uniform: scalar copies keep the table resources in
