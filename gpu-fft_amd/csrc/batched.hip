@@ -1098,7 +1098,11 @@ __device__ __forceinline__ void dispatch_s(cplx<T>* lds, const BArgs& ba, const 
 // those still hold items is one read of all counters by the first wavefront: an
 // atomic on every queue by every workgroup, all on one cache line, took 11 us
 // at the end of a launch (3 products FP64 50 -> 39 us, 700 FP32 1006 -> 957).
-// Index of the next item, -1 once all queues are exhausted.  sh: the index, and
+// Index of the next item, of the home queue, then of the others; -1 once all are
+// exhausted.  Which of them still hold items is one read of all counters by the
+// first wavefront: an atomic on every queue by every workgroup, all on one cache
+// line, took 11 us at the end of a launch (3 products FP64 50 -> 39 us, 700 FP32
+// 1006 -> 953).  sh: the index, and
 // whether the home queue is known to be exhausted (set to 0 by the first
 // wavefront before the first call; in LDS, as registers held across the items
 // cost the FP32 kernels spills: 4096 products on the smaller tile 4.81 -> 5.03 ms).
