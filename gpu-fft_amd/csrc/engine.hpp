@@ -94,9 +94,13 @@ __device__ __forceinline__ void group_stages_derived(cplx<T>* v, const PassArgs<
 #pragma unroll
         for (int t = 0; t < (1 << s); t++) {
             cplx<T> w = base;
-            if (t == 1 && s == 1) {
-                // times exp(+-i pi/2), exact: forward chains use the roots,
-                // inverse chains (Gentleman-Sande) their conjugates
+            if (TW && t == 1 && s == 1) {
+                // times tab[1] = exp(+-i pi/2), exact
+                const T sg = wc[1].y < T(0) ? T(-1) : T(1);
+                w = mk<T>(-sg * base.y, sg * base.x);
+            } else if (t == 1 && s == 1) {
+                // the same of the plans' own tables: forward chains use the
+                // roots, inverse chains (Gentleman-Sande) their conjugates
                 w = mode_is_ct(MODE) ? mk<T>(-base.y, base.x) : mk<T>(base.y, -base.x);
             } else if (t > 0) {
                 w = base * wc[TW ? t : (1 << s) + t];

@@ -10,6 +10,11 @@
 // p + 2^b differ by twist[2^b], so the stage on bit b takes root[..] twist[2^b],
 // formed once per workgroup.
 //
+// The caller may pass the tables of the other direction.  The stages derive
+// quarter turns for exp(+2 pi i ..) roots, so conjugate roots run them on
+// conjugates: conj_if on the twiddles, the gathered inputs and the outputs
+// (the coefficients of the gather are the table's own).
+//
 // Workgroups are persistent, one per CU, and load the next transform while they
 // work on the current one (why, see product.hpp).  FFNT N = 2^16, 512
 // transforms: 127 -> 95 us (4.2 -> 5.7 TB/s in and out); R_R of 2^16 points, 128
@@ -23,6 +28,16 @@
 #include "subfft.hpp"
 
 namespace gfa {
+
+// conj(z) if flip is the sign bit, z if it is 0
+__device__ __forceinline__ cplx<double> conj_if(cplx<double> z, unsigned flip)
+{
+    u32x2 y;
+    __builtin_memcpy(&y, &z.y, 8);
+    y[1] ^= flip;
+    __builtin_memcpy(&z.y, &y, 8);
+    return z;
+}
 
 template <int SB, bool FOLD>
 __global__ __launch_bounds__(512, 2) void forward13_kernel(OneArgs<double> o)
@@ -60,11 +75,13 @@ __global__ __launch_bounds__(512, 2) void forward13_kernel(OneArgs<double> o)
 #pragma unroll
     for (int j = 0; j < Q; j++) C[j] = uniform(C[j]);
 
+    // tab[1] = exp(+-i pi/2)
+    const unsigned flip = o.tab[1].y < 0.0 ? 0x80000000u : 0u;
     auto entry = [&](auto qc, auto rhoc, int H, int e) {
         constexpr int lo = decltype(qc)::value, rho = decltype(rhoc)::value;
         cplx<double> w = o.tab[lead_entry<rho>(H + (o.nega ? 1 << (n - lo - rho) : 0), e)];
         if constexpr (FOLD) w = w * o.twist[1 << (lo + rho - 1 - lead_stage<rho>(e))];
-        return w;
+        return conj_if(w, flip);
     };
     W w;
     w.table = table;
@@ -79,6 +96,8 @@ __global__ __launch_bounds__(512, 2) void forward13_kernel(OneArgs<double> o)
     cplx<double> v[16], next[16];
     first.end(x0, L, tid, v, C);
     arrived(v);
+#pragma unroll
+    for (int e = 0; e < 16; e++) v[e] = conj_if(v[e], flip);
     Gather13<SB, FOLD> gather;
     __syncthreads();
     for (; t < o.batch; t += step) {
@@ -105,9 +124,9 @@ __global__ __launch_bounds__(512, 2) void forward13_kernel(OneArgs<double> o)
         cplx<double>* dst = static_cast<cplx<double>*>(o.dst) + t * o.dst_stride + hi;
 #pragma unroll
         for (int e = 0; e < 16; e++)
-            stc_nt(&at(dst + WaveMap<S, 2>::elem(e), WaveMap<S, 2>::ins(tid)), v[e]);
+            stc_nt(&at(dst + WaveMap<S, 2>::elem(e), WaveMap<S, 2>::ins(tid)), conj_if(v[e], flip));
 #pragma unroll
-        for (int e = 0; e < 16; e++) v[e] = next[e];
+        for (int e = 0; e < 16; e++) v[e] = conj_if(next[e], flip);
     }
 }
 
