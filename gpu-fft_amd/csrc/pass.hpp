@@ -195,7 +195,7 @@ template <typename T, int MODE> __device__ __forceinline__ void butterfly(cplx<T
 }
 
 // i sg w: a quarter turn in the table's direction (sg = +1 for a table of
-// exp(+2 pi i ..), -1 for its conjugate)
+// exp(+2 pi i ..), -1 for its conjugate; of the table of k-th powers, k odd: i^k)
 template <typename T> __device__ __forceinline__ cplx<T> quarter(cplx<T> w, T sg)
 {
     return mk<T>(-sg * w.y, sg * w.x);
@@ -444,8 +444,12 @@ __global__ __launch_bounds__((1 << pass_tile<T>(COL, K)) >> PASS_E, 4) void radi
     Shape g;
     g.init(blockIdx.x, a.n, a.blo);
     const rsrc_t tab = make_rsrc(a.tab);
-    // the table's direction: tab[1] = exp(+-i pi/2) (standard), exp(+-i pi/4) (special)
-    const T sg = (K > 1 && a.tab[1].y < T(0)) ? T(-1) : T(1);
+    // the table's direction (Twid): tab[1] is i^k (standard), exp(k i pi/4) (special)
+    T sg = T(1);
+    if constexpr (K > 1) {
+        const cplx<T> w1 = a.tab[1];
+        if ((w1.y < T(0)) != (mode_special(MODE) && w1.x < T(0))) sg = T(-1);
+    }
     // special step at bit 0: its entries are uniform, read here (ahead of any
     // barrier) so that they are scalar loads
     cplx<T> low[16];
