@@ -237,12 +237,22 @@ int run_f64(const gpufft_polymul_plan_s* plan, const double* a, const double* b,
 }
 
 // ---- products without allocation ----
-// Static device scratch of gpufft_polymul_f64_noalloc: the merged root table
-// (written by every call) and the sub-problem results of products split over
-// several workgroups, room for 64 MiB of them beside the largest table.
-// Each device holds its own copy from module load until the process ends;
-// calls that overlap in time on one device share it and race.
-constexpr size_t NOALLOC_TABLE_BYTES = ((size_t)1 << 20) + 1024;  // n = 16, SB = 3: 2^16 + 64 entries
+// Static device scratch of gpufft_polymul_f64_noalloc: the merged root tables
+// (every call writes its ring's) and the sub-problem results of products split
+// over several workgroups (64 MiB).  Each device holds its own copy from module
+// load until the process ends.  No entry of a table depends on which ring's call
+// wrote it: unsplit rings take the first roots of the longest table, and the
+// split ones, whose residue powers stand behind the roots, have a table each.
+// So calls that overlap in time on one device race for the sub-problem results
+// only (split rings).
+// First entry of the split table of 2^n points (n = 13: the end of them all).
+constexpr size_t noalloc_table(int n)
+{
+    size_t at = 0;
+    for (int k = F64_MAX_S + MAX_SB; k > n; k--) at += product_table_entries(k, k - F64_MAX_S);
+    return at;
+}
+constexpr size_t NOALLOC_TABLE_BYTES = (sizeof(cplx<double>) * noalloc_table(F64_MAX_S) + 4095) / 4096 * 4096;
 constexpr size_t NOALLOC_BYTES = NOALLOC_TABLE_BYTES + ((size_t)64 << 20);
 static __device__ __align__(256) unsigned char scratch[NOALLOC_BYTES];
 
@@ -563,7 +573,7 @@ int gpufft_polymul_f64_noalloc(const double* a, const double* b, double* out, in
     pl.ka = pl.kb = 1;
     pl.S = std::min(n, F64_MAX_S);
     pl.SB = n - pl.S;
-    pl.root = base;
+    pl.root = (cplx<double>*)base + (pl.SB > 0 ? noalloc_table(n) : 0);
     // the sub-problem results of one launch must fit the rest of the array:
     // the batch runs in launches of at most that many products
     const size_t per_product = pl.SB > 0 ? (sizeof(cplx<double>) << n) : 0;
@@ -571,7 +581,7 @@ int gpufft_polymul_f64_noalloc(const double* a, const double* b, double* out, in
     pl.max_batch = per_product ? (int)std::min<size_t>(room / per_product, (size_t)batch) : batch;
     pl.scratch = pl.SB > 0 ? (void*)((unsigned char*)base + NOALLOC_TABLE_BYTES) : nullptr;
     pl.scratch_bytes = pl.SB > 0 ? room : 0;
-    // the merged roots: rewritten by every call (a kernel, so the call can be
+    // the merged roots: written by every call (a kernel, so the call can be
     // captured into a graph), ahead of the product kernels on `st`
     if (int s = launch_product_table(pl.root, n, pl.SB, st, who)) return s;
     return run_f64(&pl, a, b, out, batch, GPUFFT_PHASE_ALL, st, who);

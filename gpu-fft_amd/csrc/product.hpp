@@ -51,7 +51,7 @@ namespace gfa {
 struct ProductArgs {
     int n;      // log2 of the complex length L
     int batch;  // products in this launch
-    const cplx<double>* w;  // merged roots W (L entries), then zeta_q^j at [L + q Q + j]
+    const cplx<double>* w;  // merged roots W (L entries), for SB > 0 then zeta_q^j at [L + q Q + j]
     const double* a;
     const double* b;
     double* out;            // SB = 0: [batch][2L]
@@ -310,17 +310,18 @@ template <int SB> __global__ __launch_bounds__(256) void combine_f64_kernel(Comb
     }
 }
 
-// Fills W (2^n entries) and the residue powers zeta_q^j (2^SB x 2^SB) behind it.
+// Fills W (2^n entries, the first ones of every longer W) and, for SB > 0, the
+// residue powers zeta_q^j (2^SB x 2^SB) behind it.
 __global__ void product_table_kernel(cplx<double>* w, int n, int SB)
 {
     const int k = blockIdx.x * 256 + threadIdx.x;
     const int L = 1 << n, Q = 1 << SB;
-    if (k >= L + Q * Q) return;
+    if (k >= L + (SB > 0 ? Q * Q : 0)) return;
     // angle 2 pi num / den, exact
     double num = 0.0, den = 1.0;
     if (k >= L) {
         const int q = (k - L) >> SB, j = (k - L) & (Q - 1);
-        const int r = SB ? (int)(__brev((unsigned)q) >> (32 - SB)) : 0;
+        const int r = (int)(__brev((unsigned)q) >> (32 - SB));
         num = (double)((1 + 4 * r) * j);
         den = 4.0 * Q;
     } else if (k > 0) {

@@ -7,8 +7,12 @@
 
 namespace gfa {
 
-// Entries of the merged root table: 2^n roots, 4^SB residue powers.
-inline size_t product_table_entries(int n, int SB) { return ((size_t)1 << n) + ((size_t)1 << (2 * SB)); }
+// Entries of the merged root table: 2^n roots and, of split products, 4^SB
+// residue powers.
+constexpr size_t product_table_entries(int n, int SB)
+{
+    return ((size_t)1 << n) + (SB > 0 ? (size_t)1 << (2 * SB) : 0);
+}
 
 // Workgroups of a persistent launch of which `resident` share a CU: what the
 // CUs hold at once, if there is as much work.

@@ -246,16 +246,18 @@ int gpufft_polymul_i32_phases(gpufft_polymul_plan plan, const int32_t* a, const 
  * harnesses that forbid hipMalloc).  The caller passes the inputs, the
  * output and the four FFNT tables of ring N = 2^ring_power (N/2 entries
  * each, the layouts GPU_FFNT takes: twist, untwist, root and inverse root,
- * e.g. from gpufft_generate_table_f64; the kernels take their roots from a
- * table that the call generates, so these are only checked for NULL); the
- * library uses a static device array of 65 MiB (per device, held until the
- * process ends) for that table and the sub-problem results, so the batch
- * runs in launches of at most 64 MiB / (8 N) products for ring_power >= 15.  ring_power 7..17
- * (else GPUFFT_ERR_INVALID_ARGUMENT); a, b, out: double [batch][N]; out is
- * the unrounded product mod X^N+1, equal to gpufft_polymul_f64's.  Calls
- * that overlap in time on one device share the array and race; calls on one
- * stream are ordered.  Only kernels are enqueued (no memset, no
- * allocation), so a call can be captured into a HIP graph. */
+ * e.g. from gpufft_generate_table_f64; the kernels take their roots from
+ * tables that the call generates, so these are only checked for NULL); the
+ * library uses a static device array of 66 MiB (per device, held until the
+ * process ends) for those tables and the sub-problem results, so the batch
+ * runs in launches of at most 64 MiB / (8 N) products for ring_power >= 15.
+ * ring_power 7..17 (else GPUFFT_ERR_INVALID_ARGUMENT); a, b, out: double
+ * [batch][N]; out is the unrounded product mod X^N+1, equal to
+ * gpufft_polymul_f64's.  Calls of ring_power >= 15 that overlap in time on
+ * one device share the sub-problem results and race; smaller rings use only
+ * the tables, whose values are the same in every call.  Calls on one stream
+ * are ordered.  Only kernels are enqueued (no memset, no allocation), so a
+ * call can be captured into a HIP graph. */
 int gpufft_polymul_f64_noalloc(const double* a, const double* b, double* out, int ring_power,
                                int batch, const void* twist, const void* untwist,
                                const void* root_table, const void* inv_root_table, void* stream);
