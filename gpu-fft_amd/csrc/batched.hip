@@ -1094,24 +1094,20 @@ __device__ __forceinline__ void dispatch_s(cplx<T>* lds, const BArgs& ba, const 
     }
 }
 
-// The workgroup's items: its home queue's, then the other queues'.  Which of
-// those still hold items is one read of all counters by the first wavefront: an
-// atomic on every queue by every workgroup, all on one cache line, took 11 us
-// at the end of a launch (3 products FP64 50 -> 39 us, 700 FP32 1006 -> 957).
-// Index of the next item, of the home queue, then of the others; -1 once all are
-// exhausted.  Which of them still hold items is one read of all counters by the
-// first wavefront: an atomic on every queue by every workgroup, all on one cache
-// line, took 11 us at the end of a launch (3 products FP64 50 -> 39 us, 700 FP32
-// 1006 -> 953).  sh: the index, and
-// whether the home queue is known to be exhausted (set to 0 by the first
-// wavefront before the first call; in LDS, as registers held across the items
-// cost the FP32 kernels spills: 4096 products on the smaller tile 4.81 -> 5.03 ms).
+// Index of the workgroup's next item: its home queue's, then the other queues';
+// -1 once all are exhausted.  Which of the others still hold items is one read
+// of all counters by the first wavefront: an atomic on every queue by every
+// workgroup, all on one cache line, took 11 us at the end of a launch (3
+// products FP64 50 -> 39 us, 700 FP32 1006 -> 953).  sh: the index, and whether
+// the home queue is known to be exhausted (0 and a barrier before the first
+// call; in LDS, as registers held across the items cost the FP32 kernels
+// spills: 4096 products on the smaller tile 4.81 -> 5.03 ms).
 __device__ __forceinline__ int next_item(const BArgs& ba, int tid, int* sh)
 {
     if (tid < 64) {
         const int home = (int)(blockIdx.x % NQ);
         int got = -1, x = home;
-        bool look = sh[1] != 0;
+        bool look = __builtin_amdgcn_readfirstlane(sh[1]) != 0;
         for (;;) {
             if (look) {
                 bool has = false;
@@ -1159,6 +1155,7 @@ void batched_kernel(BArgs ba)
     __shared__ int sh_last;
     const int tid = threadIdx.x;
     if (tid == 0) sh_item[1] = 0;
+    __syncthreads();
     for (;;) {
         const int it = next_item(ba, tid, sh_item);
         if (it < 0) break;
