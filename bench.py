@@ -41,7 +41,8 @@ def parse():
     p.add_argument("--a-center", type=int, default=19,
                    help="FP32 split of a - 2^c plus the exact 2^c (J b) limb (0: split a as is)")
     p.add_argument("--cpu-seconds", type=float, default=10.0)
-    p.add_argument("--rb-f64", type=int, default=0, help="radix bits of the FP64 kernel (0: tune)")
+    p.add_argument("--rb-f64", type=int, default=0,
+                   help="radix bits setting of the FP64 plan (0: the default; one kernel serves all)")
     p.add_argument("--rb-f32", type=int, default=0, help="radix bits of the FP32 kernel (0: tune)")
     p.add_argument("--e-f32", type=int, default=0,
                    help="log2 points per thread of the FP32 kernel, 5 or 4 (0: tune)")
@@ -760,7 +761,7 @@ def main():
         if "f64" in forms:
             plan = G.PolymulPlan(rp, G.PREC_F64, max_batch=batch, stream=sid)
             out = torch.empty(batch * N, dtype=torch.float64, device=dev)
-            tune = tune_radix(plan, [args.rb_f64] if args.rb_f64 else [3, 4],
+            tune = tune_radix(plan, [args.rb_f64 or 4],  # one kernel at every setting
                               lambda: plan.multiply_f64(a64, b64, out, batch, stream=sid),
                               stream, args.steps)
             plan.radix_bits = min(tune, key=tune.get)

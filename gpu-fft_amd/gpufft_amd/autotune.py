@@ -6,7 +6,7 @@ plans for the same workload reuse the choice without timing again.
 
 Tuned knobs (each changes speed only; results are the same up to rounding,
 and rounded products are identical):
-  polymul plans  radix bits of the LDS steps (gpufft_polymul_plan_set_radix_bits)
+  polymul plans  FP32 split: radix bits of the LDS steps (gpufft_polymul_plan_set_radix_bits)
   batched plans  radix bits and persistent grid size (gpufft_batched_plan_set_tuning)
 
 The database is $GPUFFT_AMD_TUNING_DB, else ~/.cache/gpufft_amd/tuning.json.
@@ -109,7 +109,10 @@ def tune(key, candidates, apply, run, stream, reps=5, use_db=True, db_file=None)
 
 
 def tune_polymul(plan, run, stream, key=None, reps=5, use_db=True, db_file=None):
-    rbs = (3, 4) if plan.precision == 0 else (3, 4, 5)
+    """FP32-split plans: radix 2^3 to 2^5.  FP64 plans run the same kernel at
+    every setting and keep the default."""
+    from . import PREC_F64
+    rbs = (4,) if plan.precision == PREC_F64 else (3, 4, 5)
     key = key or signature("polymul", plan.ring_power, plan.precision)
     return tune(key, [(r,) for r in rbs], lambda c: setattr(plan, "radix_bits", c[0]), run, stream,
                 reps, use_db, db_file)
