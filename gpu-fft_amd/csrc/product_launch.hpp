@@ -14,15 +14,21 @@ constexpr size_t product_table_entries(int n, int SB)
     return ((size_t)1 << n) + (SB > 0 ? (size_t)1 << (2 * SB) : 0);
 }
 
-// Workgroups of a persistent launch of which `resident` share a CU: what the
-// CUs hold at once, if there is as much work.
-inline int persistent_grid(long long items, int resident)
+// Compute units of the current device.
+inline int device_cus()
 {
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 64)
         cus = 256;
-    return (int)std::min<long long>(items, (long long)cus * resident);
+    return cus;
+}
+
+// Workgroups of a persistent launch of which `resident` share a CU: what the
+// CUs hold at once, if there is as much work.
+inline int persistent_grid(long long items, int resident)
+{
+    return (int)std::min<long long>(items, (long long)device_cus() * resident);
 }
 
 int launch_product_table(void* w, int n, int SB, hipStream_t st, const char* who);

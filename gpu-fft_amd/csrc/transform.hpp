@@ -10,6 +10,7 @@
 #include "engine.hpp"
 #include "oneshot.hpp"
 #include "passes.hpp"
+#include "product_launch.hpp"
 #include "status.hpp"
 
 namespace gfa {
@@ -168,21 +169,21 @@ template <typename T, int SB> TopFn<T> select_top_sb(int sk)  // SB = 2..4
 //   FP64 forward: few transforms (the chain's workgroups are smaller): FFNT of
 //     2^16 points x 2: 12.4 / 17.5, x 8 17.0 / 17.8, x 16 21.1 / 18.1; of 2^15
 //     x 2 11.6 / 12.3, x 8 13.6 / 12.7; R_R of 2^16 x 2 11.6 / 12.5, x 8 15.8 /
-//     12.8.  FFNT of 2^16 points has 8 workgroups to a transform: past 32
-//     transforms a second, emptier wave: x 36 32.8 / 40.5, x 64 43.3 / 43.8,
-//     x 128 85 / 74.
+//     12.8.  FFNT of 2^16 points has 8 workgroups to a transform, one to a CU: a
+//     second wave (33 .. 64 transforms on 256 CUs) is emptier than the chain's
+//     last: x 36 32.8 / 40.5, x 64 43.3 / 43.8, x 128 85 / 74.
 //   FP32 inverse: R_R 2^15 x 128 17.3 / 20.7, x 1024 92 / 108; FFNT 2^15 points
 //     x 256 52 / 61, x 1 10.5 / 14.0, 2^16 x 1 10.7 / 14.9.
 //   FP32 forward up to 2^20 points in the launch (FFNT 2^15 x 16: 11.3 / 14.8, x
 //     32 14.1 / 14.9, x 64 19.1 / 15.1; R_R 2^16 x 16 13.4 / 13.6, x 32 20 / 13.6;
 //     R_R 2^15 x 16 10.5 / 12.4, x 32 13.3 / 12.6), and FFNT of 2^17 points (x 2
 //     10.7 / 22.5, x 64 51 / 60).
-template <typename T> bool prefer_passes(bool forward, int n, int batch, bool fold)
+template <typename T> bool prefer_passes(bool forward, int n, int batch, bool fold, int cus)
 {
     const long long points = (long long)batch << n;
     if constexpr (sizeof(T) == 8) {
         if (!forward) return false;
-        if (n == 16) return batch <= (fold ? 8 : 2) || (fold && batch > 32 && batch <= 64);
+        if (n == 16) return batch <= (fold ? 8 : 2) || (fold && 8LL * batch > cus && 8LL * batch <= 2LL * cus);
         return n == 15 && fold && batch <= 2;
     }
     if (!forward || (n == 17 && fold)) return true;
@@ -199,7 +200,8 @@ bool run_oneshot(int mode, int n, int batch, int nega, const cplx<T>* tab,
     constexpr int S = OneCfg<T>::S, E = OneCfg<T>::E, RB = OneCfg<T>::RB;
     const int SB = n - S;
     if (SB < 1 || SB > 3) return false;
-    if (prefer_passes<T>(mode == MODE_STD_FWD, n, batch, io.lk == LD_FOLD)) return false;
+    const int cus = device_cus();
+    if (prefer_passes<T>(mode == MODE_STD_FWD, n, batch, io.lk == LD_FOLD, cus)) return false;
     OneArgs<T> a{};
     a.n = n;
     a.batch = batch;
@@ -226,7 +228,7 @@ bool run_oneshot(int mode, int n, int batch, int nega, const cplx<T>* tab,
         // 32: 15.7 against 13.4, x 64 17.9 against 17.5)
         bool launched = false;
         if constexpr (sizeof(T) == 8) {
-            launched = blocks > 256;
+            launched = blocks > cus;
             if (launched) launch_forward13(a, SB, io.lk == LD_FOLD, stream);
         }
         if (!launched) {

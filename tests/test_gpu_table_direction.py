@@ -14,7 +14,8 @@ pytestmark = pytest.mark.gpu
 # batches on both sides of the lines between the kernels, 256 compute units
 FORWARD = [("f64", 13, 3), ("f64", 14, 1), ("f64", 14, 128), ("f64", 14, 130), ("f64", 15, 2),
            ("f64", 15, 3), ("f64", 15, 64), ("f64", 15, 65), ("f64", 16, 2), ("f64", 16, 3),
-           ("f64", 16, 8), ("f64", 16, 9), ("f64", 16, 33), ("f64", 16, 65), ("f64", 17, 2),
+           ("f64", 16, 8), ("f64", 16, 9), ("f64", 16, 32), ("f64", 16, 33), ("f64", 16, 64),
+           ("f64", 16, 65), ("f64", 17, 2),
            ("f32", 14, 3), ("f32", 15, 16), ("f32", 15, 17), ("f32", 15, 33), ("f32", 16, 16),
            ("f32", 16, 17), ("f32", 17, 8), ("f32", 17, 9)]
 
@@ -34,10 +35,12 @@ def _tables(kind, nega, L, prec):
 
 
 @pytest.mark.parametrize("kind,nega,which", [("r2r", 0, "root"), ("r2r", 1, "root"), ("ffnt", 0, "both"),
-                                             ("ffnt", 0, "root")])
+                                             ("ffnt", 0, "root"), ("r2r", 0, "none"), ("r2r", 1, "none"),
+                                             ("ffnt", 0, "none")])
 @pytest.mark.parametrize("prec,n,batch", FORWARD)
 def test_forward_with_inverse_tables(prec, n, batch, kind, nega, which):
-    """which: both tables of the other direction, or the root table alone."""
+    """which: both tables of the other direction, the root table alone, or
+    none (the forward's own, on both sides of the same lines)."""
     import torch
     G = _g()
     L = 1 << n
@@ -47,7 +50,7 @@ def test_forward_with_inverse_tables(prec, n, batch, kind, nega, which):
     rows = sorted({0, batch // 2, batch - 1})
     some = np.concatenate([real[k * R:(k + 1) * R] for k in rows])
     fwd, inv = _tables(kind, nega, L, prec)
-    twist, root = (inv if which == "both" else fwd)[0], inv[1]
+    twist, root = (inv if which == "both" else fwd)[0], (fwd if which == "none" else inv)[1]
     dt = torch.empty(batch * L, dtype=torch.complex128 if prec == "f64" else torch.complex64, device="cuda")
     if kind == "r2r":
         rp = G.X_N_PLUS if nega else G.X_N_MINUS
