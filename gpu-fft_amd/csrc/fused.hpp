@@ -276,12 +276,11 @@ __device__ __forceinline__ void top_gs(cplx<T>* y, const ProdArgs<T>& a, int q)
 
 // Gathers the sub-problem's input into LDS: fold + twist + row q of the top
 // network for every position c < 2^S, then the HB-bit top step (top_ct).
-// ones: the operand is the all-ones polynomial J (no loads); center: the
-// limb form splits x - center.
+// center: the limb form splits x - center.
 template <typename T, int S, int SB, int E, int PL, int HB>
 __device__ __forceinline__ void load_sub(cplx<T>* lds, const ProdArgs<T>& a, rsrc_t x,
                                          const cplx<T>* tws, int w, int limb, int k, long long o,
-                                         int center, bool ones, const cplx<T>* C, int q, int tid)
+                                         int center, const cplx<T>* C, int q, int tid)
 {
     constexpr int NT = (1 << S) >> E;
     constexpr int Q = 1 << SB;
@@ -298,17 +297,9 @@ __device__ __forceinline__ void load_sub(cplx<T>* lds, const ProdArgs<T>& a, rsr
         for (int m = 0; m < NP; m++) {
             const int c0 = (tid + (g0 + m * NGH) * NT) * V;
             T re[Q][V], im[Q][V];
-            if (ones) {
 #pragma unroll
-                for (int j = 0; j < Q; j++)
-#pragma unroll
-                    for (int v = 0; v < V; v++) re[j][v] = im[j][v] = T(1);
-            } else {
-#pragma unroll
-                for (int j = 0; j < Q; j++)
-                    prod_input_vec<T, PL, V>(x, L, w, limb, k, o, center, (j << S) | c0, re[j],
-                                             im[j]);
-            }
+            for (int j = 0; j < Q; j++)
+                prod_input_vec<T, PL, V>(x, L, w, limb, k, o, center, (j << S) | c0, re[j], im[j]);
 #pragma unroll
             for (int v = 0; v < V; v++) {
                 T ax = T(0), ay = T(0);
@@ -357,9 +348,11 @@ __device__ __forceinline__ void last_forward_step(const cplx<T>* lds, const Pass
     }
 }
 
-template <typename T, int S, int SB, int E, int PL, int RB>
-__global__ __launch_bounds__((1 << S) >> E) void product_sub_kernel(ProdArgs<T> a)
+template <int S, int SB, int E, int RB>
+__global__ __launch_bounds__((1 << S) >> E) void product_sub_kernel(ProdArgs<float> a)
 {
+    using T = float;
+    constexpr int PL = PL_FOLD_LIMB;
     constexpr int TILE = 1 << S;
     constexpr int EPT = 1 << E;
     constexpr int NT = TILE / EPT;
@@ -417,7 +410,7 @@ __global__ __launch_bounds__((1 << S) >> E) void product_sub_kernel(ProdArgs<T> 
         int t = tid;
         asm volatile("" : "+v"(t));
         __syncthreads();
-        load_sub<T, S, SB, E, PL, HB>(lds, a, xb, tws, a.wb, jb, a.kb, a.ob, 0, false, C, q, t);
+        load_sub<T, S, SB, E, PL, HB>(lds, a, xb, tws, a.wb, jb, a.kb, a.ob, 0, C, q, t);
         run_steps_ct<T, MODE_STD_FWD, E, NT, S, RB, FS0, NST - 1>(lds, pf, g, t, a.wc);
         last_forward_step<T, E, RB, NT>(lds, pf, g, t, breg, a.wc);
         for (int ia = 0; ia < nla; ia++) {
@@ -428,7 +421,7 @@ __global__ __launch_bounds__((1 << S) >> E) void product_sub_kernel(ProdArgs<T> 
             const bool jl = ia >= a.ka;
             if (!jl) {
                 load_sub<T, S, SB, E, PL, HB>(lds, a, xa, tws, a.wa, ia, a.ka, a.oa,
-                                              a.ca ? (1 << a.ca) : 0, false, C, q, u);
+                                              a.ca ? (1 << a.ca) : 0, C, q, u);
                 run_steps_ct<T, MODE_STD_FWD, E, NT, S, RB, FS0, NST - 1>(lds, pf, g, u,
                                                                                a.wc);
             }

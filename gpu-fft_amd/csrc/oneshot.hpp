@@ -98,7 +98,7 @@ __global__ __launch_bounds__((1 << S) >> E) void fwd_sub_kernel(OneArgs<T> o)
     top_row_coeffs<T, SB, TWIST>(a, q, C);
     const rsrc_t xa = make_rsrc(reinterpret_cast<const T*>(o.src) + t * o.src_stride);
     __syncthreads();
-    load_sub<T, S, SB, E, PL, HB>(lds, a, xa, tws, 0, 0, 1, 0, 0, false, C, q, tid);
+    load_sub<T, S, SB, E, PL, HB>(lds, a, xa, tws, 0, 0, 1, 0, 0, C, q, tid);
     run_steps_ct<T, MODE_STD_FWD, E, NT, S, RB, FS0, NST, true>(lds, pf, g, tid, o.tab);
     cplx<T>* dst = reinterpret_cast<cplx<T>*>(o.dst) + t * o.dst_stride + ((long long)q << S);
 #pragma unroll 4

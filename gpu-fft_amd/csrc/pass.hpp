@@ -112,11 +112,6 @@ template <int Q, int RHO> struct StepMap {
         return ins((e >> RHO) << NTL) | ((e & ((1 << RHO) - 1)) << Q);
     }
 };
-// consecutive lanes on consecutive elements
-struct LinearMap {
-    static __host__ __device__ constexpr int ins(int g) { return g; }
-    template <int NTL> static __host__ __device__ constexpr int elem(int e) { return e << NTL; }
-};
 // CKKS: lanes run over natural (not bit-reversed) positions; with K < LT the
 // tile holds 2^(LT-K) blocks whose reversed block numbers are consecutive.
 template <int K, int LT> struct ReverseMap {

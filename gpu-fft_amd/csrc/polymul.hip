@@ -52,7 +52,7 @@ constexpr int F32_MAX_S = 14;  // 2^14 floats complex = 128 KiB of LDS
 constexpr int MAX_SB = 3;
 constexpr int F64_E = 4;   // FP64 plans: log2 points per thread
 
-template <typename T> using ProdKernel = void (*)(ProdArgs<T>);
+using ProdKernel = void (*)(ProdArgs<float>);
 
 // Zero fill by a kernel rather than hipMemsetAsync, so that a caller may
 // capture the call into a HIP graph.
@@ -71,19 +71,19 @@ __global__ void fill_ones(float* p, long long n)
 // Whether the product kernel exists for a sub-problem of 2^S points, 2^E
 // points per thread and radix-2^RB steps: the thread's groups of V loaded
 // positions must hold the 2^(S mod RB) partners of the register top step.
-template <typename T, int S, int E, int PL, int RB> constexpr bool prod_ok()
+template <int S, int E, int RB> constexpr bool prod_ok()
 {
     constexpr int HB = S % RB;
-    constexpr int V = in_vec<T, PL, E, HB>();
+    constexpr int V = in_vec<float, PL_FOLD_LIMB, E, HB>();
     return RB <= E && S > E && ((1 << E) / V) / (1 << HB) >= 1;
 }
 
 // FP32 split, 2^E points per thread: 2^(S-E) threads per workgroup
-template <int RB, int E> ProdKernel<float> prod_kernel_rb(int S, int SB)
+template <int RB, int E> ProdKernel prod_kernel_rb(int S, int SB)
 {
 #define GFA_PK(SS, BB)                                                 \
-    if constexpr (prod_ok<float, SS, E, PL_FOLD_LIMB, RB>())           \
-        if (S == SS && SB == BB) return &product_sub_kernel<float, SS, BB, E, PL_FOLD_LIMB, RB>;
+    if constexpr (prod_ok<SS, E, RB>())                                \
+        if (S == SS && SB == BB) return &product_sub_kernel<SS, BB, E, RB>;
     GFA_PK(7, 0)
     GFA_PK(8, 0)
     GFA_PK(9, 0)
@@ -101,7 +101,7 @@ template <int RB, int E> ProdKernel<float> prod_kernel_rb(int S, int SB)
 
 // radix bits per LDS step 3..5, points per thread 2^e: 32 or 16; both chosen
 // per plan
-template <int E> ProdKernel<float> prod_kernel_e(int S, int SB, int rb)
+template <int E> ProdKernel prod_kernel_e(int S, int SB, int rb)
 {
     switch (rb) {
         case 3: return prod_kernel_rb<3, E>(S, SB);
@@ -113,7 +113,7 @@ template <int E> ProdKernel<float> prod_kernel_e(int S, int SB, int rb)
     }
 }
 
-ProdKernel<float> prod_kernel(int S, int SB, int rb, int e)
+ProdKernel prod_kernel(int S, int SB, int rb, int e)
 {
     if (e == 5) return prod_kernel_e<5>(S, SB, rb);
     if (e == 4) return prod_kernel_e<4>(S, SB, rb);
@@ -163,26 +163,25 @@ void release(gpufft_polymul_plan_s* pl)
 int launch_split(const gpufft_polymul_plan_s* pl, const int32_t* a, const int32_t* b, int batch,
                  hipStream_t st, const char* who)
 {
-    using T = float;
-    ProdArgs<T> pa{};
+    ProdArgs<float> pa{};
     pa.n = pl->n;
     pa.S = pl->S;
     pa.batch = batch;
     pa.nega = 0;
-    pa.tab = (const cplx<T>*)pl->root;
-    pa.itab = (const cplx<T>*)pl->iroot;
-    pa.twist = (const cplx<T>*)pl->twist;
-    pa.untwist = (const cplx<T>*)pl->untwist;
-    pa.wc = (const cplx<T>*)pl->wc;
-    pa.wci = (const cplx<T>*)pl->wci;
+    pa.tab = (const cplx<float>*)pl->root;
+    pa.itab = (const cplx<float>*)pl->iroot;
+    pa.twist = (const cplx<float>*)pl->twist;
+    pa.untwist = (const cplx<float>*)pl->untwist;
+    pa.wc = (const cplx<float>*)pl->wc;
+    pa.wci = (const cplx<float>*)pl->wci;
     pa.a = a;
     pa.b = b;
     pa.in_stride = 2LL << pl->n;
-    pa.scratch = (cplx<T>*)pl->scratch;
+    pa.scratch = (cplx<float>*)pl->scratch;
     pa.wa = pl->wa;
     pa.ka = pl->ka;
     pa.ca = pl->ca;
-    pa.jspec = (const cplx<T>*)pl->jspec;
+    pa.jspec = (const cplx<float>*)pl->jspec;
     pa.wb = pl->wb;
     pa.kb = pl->kb;
     auto offset = [](int w, int k) {
@@ -192,7 +191,7 @@ int launch_split(const gpufft_polymul_plan_s* pl, const int32_t* a, const int32_
     };
     pa.oa = pl->ka > 1 ? offset(pl->wa, pl->ka) : 0;
     pa.ob = pl->kb > 1 ? offset(pl->wb, pl->kb) : 0;
-    ProdKernel<T> k = prod_kernel(pl->S, pl->SB, pl->rb, pl->e);
+    ProdKernel k = prod_kernel(pl->S, pl->SB, pl->rb, pl->e);
     if (!k) return fail(GPUFFT_ERR_UNSUPPORTED, std::string(who) + ": no kernel for this size");
     const int threads = (1 << pl->S) >> pl->e;
     const long long groups = ((long long)batch + 7) / 8;
