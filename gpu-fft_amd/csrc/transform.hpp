@@ -164,6 +164,9 @@ template <typename T, int SB> TopFn<T> select_top_sb(int sk)  // SB = 2..4
     return nullptr;
 }
 
+// Workgroups of a one-launch forward: transforms in groups of 8, one per XCD.
+inline long long one_blocks(int batch, int SB) { return (((long long)batch + 7) / 8 * 8) << SB; }
+
 // Where the pass chain is faster than this path (us, both sides measured, chain
 // against this path):
 //   FP64 forward: few transforms (the chain's workgroups are smaller): FFNT of
@@ -178,6 +181,13 @@ template <typename T, int SB> TopFn<T> select_top_sb(int sk)  // SB = 2..4
 //     32 14.1 / 14.9, x 64 19.1 / 15.1; R_R 2^16 x 16 13.4 / 13.6, x 32 20 / 13.6;
 //     R_R 2^15 x 16 10.5 / 12.4, x 32 13.3 / 12.6), and FFNT of 2^17 points (x 2
 //     10.7 / 22.5, x 64 51 / 60).
+//   FP32 forward of 2^16 and 2^17 points where the launch's second wave is at
+//     most a quarter full (product flow, cycled buffers: FFNT 2^16 x 66 72 -> 64,
+//     x 80 73 -> 67, R_R 2^17 x 40 66 -> 57; past that R_R 2^16 x 96 60 / 63).
+// FP64 inverse, with the product (this path against the chain): R_R 2^14 x 1 9.5 /
+// 10.9, x 256 56 / 66; 2^15 x 64 29 / 31; 2^16 x 1 11.6 / 11.2, x 8 15.0 / 15.1, x
+// 64 57 / 66, x 512 418 / 465; FFNT 2^14 points x 1 9.9 / 12.7, x 256 62 / 72; 2^16 x
+// 1 13.5 / 13.8, x 64 64 / 80, x 512 478 / 533: never the chain.
 template <typename T> bool prefer_passes(bool forward, int n, int batch, bool fold, int cus)
 {
     const long long points = (long long)batch << n;
@@ -187,7 +197,26 @@ template <typename T> bool prefer_passes(bool forward, int n, int batch, bool fo
         return n == 15 && fold && batch <= 2;
     }
     if (!forward || (n == 17 && fold)) return true;
-    return points <= (n == 15 && !fold ? 1LL << 19 : 1LL << 20);
+    const long long blocks = one_blocks(batch, n - 14);
+    return points <= (n == 15 && !fold ? 1LL << 19 : 1LL << 20) ||
+           (n >= 16 && blocks > cus && 4 * blocks <= 5LL * cus);
+}
+
+// FP64 forwards of 2^n points in one launch: the persistent form (forward.hpp)
+// instead of one workgroup per sub-problem.  It starts longer and gains from the
+// second wave of workgroups on; forward and inverse with the product, repeated
+// and with cycled buffers (us, per sub-problem -> persistent):
+//   R_R  2^14 x 136 48 -> 46, 49 -> 46, x 256 62 -> 53, 61 -> 55; 2^15 x 72 47 -> 47, 53 -> 51,
+//        x 128 62 -> 57, 64 -> 59;  2^16, eight reads of every input: x 34 50 -> 52, 57 ->
+//        59, x 72 86 -> 86, 93 -> 93, x 96 93 -> 92, 101 -> 98, x 128 126 -> 115, 132 -> 129
+//   FFNT 2^14 points x 160 52 -> 54, 57 -> 58, x 192 56 -> 57, 61 -> 61, x 224 62 -> 61, 66 ->
+//        64, x 512 144 -> 133, 151 -> 138; 2^15 x 72 54 -> 55, 63 -> 62, x 112 64 -> 62, 71 ->
+//        70, x 512 290 -> 263, 290 -> 263; 2^16 x 66 109 -> 115, 122 -> 129, x 130 182 -> 191,
+//        202 -> 208, x 512 673 -> 679 (whose buffers leave the cache while it runs)
+inline bool persistent_forward(int n, bool fold, long long blocks, int cus)
+{
+    if (n == 16) return !fold && blocks >= 3LL * cus;
+    return fold ? 2 * blocks > 3LL * cus : blocks > cus;
 }
 
 // Returns true and launches when this path covers the transform (status in
@@ -217,18 +246,14 @@ bool run_oneshot(int mode, int n, int batch, int nega, const cplx<T>* tab,
     a.do_scale = io.do_scale ? 1 : 0;
     a.scale = io.do_scale ? io.scale : mk<T>(T(1), T(0));
     if (mode == MODE_STD_FWD && io.sk == ST_CPLX && (io.lk == LD_REAL || io.lk == LD_FOLD)) {
-        const long long blocks = (((long long)batch + 7) / 8) * 8 * (1LL << SB);
+        const long long blocks = one_blocks(batch, SB);
         if (blocks > 0x7fffffffLL) {
             *status = fail(GPUFFT_ERR_INVALID_ARGUMENT, std::string(who) + ": batch too large");
             return true;
         }
-        // FP64: the persistent form past one workgroup per CU (R_R 2^14 x
-        // 512: 34.7 us against 50.8, FFNT 2^15 points x 72 26.0 against 29.5, x
-        // 512 95 against 127); up to there its longer start counts (FFNT 2^15 x
-        // 32: 15.7 against 13.4, x 64 17.9 against 17.5)
         bool launched = false;
         if constexpr (sizeof(T) == 8) {
-            launched = blocks > cus;
+            launched = persistent_forward(n, io.lk == LD_FOLD, blocks, cus);
             if (launched) launch_forward13(a, SB, io.lk == LD_FOLD, stream);
         }
         if (!launched) {
