@@ -36,6 +36,16 @@ template <typename T> __device__ __forceinline__ cplx<T> operator*(cplx<T> a, cp
     return mk<T>(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }
 
+// v with the bits of `mask` (the sign bit or 0) of its high word inverted
+__device__ __forceinline__ float flip_sign(float v, unsigned mask)
+{
+    return __uint_as_float(__float_as_uint(v) ^ mask);
+}
+__device__ __forceinline__ double flip_sign(double v, unsigned mask)
+{
+    return __hiloint2double(__double2hiint(v) ^ (int)mask, __double2loint(v));
+}
+
 // Buffer resources: a 64-bit base in scalar registers plus a 32-bit byte
 // offset per lane, so that every access costs one VGPR of address instead of
 // two, and an access beyond num_records bytes reads 0 / is dropped.

@@ -38,6 +38,7 @@ template <typename T> struct PassArgs {
     int K;       // number of bits (stages) of the sub-problem
     int nega;    // X^N+1 twiddle base (standard modes only)
     const cplx<T>* tab;  // root-of-unity table (reference layout)
+    unsigned conj;       // TW (group_stages_derived): the sign bit if tab[1] = -i, 0 if it is i
 };
 
 // Bank-conflict swizzle: permutes each aligned block of 16 elements by the
@@ -96,8 +97,7 @@ __device__ __forceinline__ void group_stages_derived(cplx<T>* v, const PassArgs<
             cplx<T> w = base;
             if (TW && t == 1 && s == 1) {
                 // times tab[1] = exp(+-i pi/2), exact
-                const T sg = wc[1].y < T(0) ? T(-1) : T(1);
-                w = mk<T>(-sg * base.y, sg * base.x);
+                w = mk<T>(flip_sign(base.y, a.conj ^ 0x80000000u), flip_sign(base.x, a.conj));
             } else if (t == 1 && s == 1) {
                 // the same of the plans' own tables: forward chains use the
                 // roots, inverse chains (Gentleman-Sande) their conjugates

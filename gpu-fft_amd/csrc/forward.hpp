@@ -32,11 +32,7 @@ namespace gfa {
 // conj(z) if flip is the sign bit, z if it is 0
 __device__ __forceinline__ cplx<double> conj_if(cplx<double> z, unsigned flip)
 {
-    u32x2 y;
-    __builtin_memcpy(&y, &z.y, 8);
-    y[1] ^= flip;
-    __builtin_memcpy(&z.y, &y, 8);
-    return z;
+    return mk<double>(z.x, flip_sign(z.y, flip));
 }
 
 template <int SB, bool FOLD>

@@ -87,6 +87,7 @@ __global__ __launch_bounds__((1 << S) >> E) void fwd_sub_kernel(OneArgs<T> o)
     pf.K = S;
     pf.nega = o.nega;
     pf.tab = o.tab;
+    pf.conj = o.tab[1].y < T(0) ? 0x80000000u : 0u;
     TileGeo g;
     g.hi_pos = q << S;
     g.blo = 0;
@@ -147,6 +148,7 @@ __global__ __launch_bounds__((1 << S) >> E) void inv_local_kernel(OneArgs<T> o)
     pi.K = S;
     pi.nega = o.nega;
     pi.tab = o.tab;
+    pi.conj = o.tab[1].y < T(0) ? 0x80000000u : 0u;
     TileGeo g;
     g.hi_pos = q << S;
     g.blo = 0;
