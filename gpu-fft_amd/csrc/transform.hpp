@@ -208,15 +208,16 @@ template <typename T> bool prefer_passes(bool forward, int n, int batch, bool fo
 // and with cycled buffers (us, per sub-problem -> persistent):
 //   R_R  2^14 x 136 48 -> 46, 49 -> 46, x 256 62 -> 53, 61 -> 55; 2^15 x 72 47 -> 47, 53 -> 51,
 //        x 128 62 -> 57, 64 -> 59;  2^16, eight reads of every input: x 34 50 -> 52, 57 ->
-//        59, x 72 86 -> 86, 93 -> 93, x 96 93 -> 92, 101 -> 98, x 128 126 -> 115, 132 -> 129
+//        59, x 48 56 -> 56, 61 -> 63, x 56 61 -> 59, 65 -> 65, x 64 66 -> 63, 69 -> 67, x 72
+//        86 -> 86, 93 -> 93, x 96 93 -> 92, 101 -> 98, x 128 126 -> 115, 132 -> 129
 //   FFNT 2^14 points x 160 52 -> 54, 57 -> 58, x 192 56 -> 57, 61 -> 61, x 224 62 -> 61, 66 ->
-//        64, x 512 144 -> 133, 151 -> 138; 2^15 x 72 54 -> 55, 63 -> 62, x 112 64 -> 62, 71 ->
-//        70, x 512 290 -> 263, 290 -> 263; 2^16 x 66 109 -> 115, 122 -> 129, x 130 182 -> 191,
-//        202 -> 208, x 512 673 -> 679 (whose buffers leave the cache while it runs)
+//        64, x 512 144 -> 133, 151 -> 138; 2^15 x 72 54 -> 55, 63 -> 62, x 96 60 -> 58, 66 -> 66,
+//        x 512 290 -> 263, 290 -> 263; 2^16 x 66 109 -> 115, 122 -> 129, x 130 182 -> 191,
+//        202 -> 208, x 512 650 -> 674, 649 -> 675
 inline bool persistent_forward(int n, bool fold, long long blocks, int cus)
 {
-    if (n == 16) return !fold && blocks >= 3LL * cus;
-    return fold ? 2 * blocks > 3LL * cus : blocks > cus;
+    if (n == 16) return !fold && 4 * blocks >= 7LL * cus;
+    return fold ? 2 * blocks >= 3LL * cus : blocks > cus;
 }
 
 // Returns true and launches when this path covers the transform (status in
