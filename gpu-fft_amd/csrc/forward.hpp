@@ -16,12 +16,13 @@
 // (the coefficients of the gather are the table's own).
 //
 // Workgroups are persistent, one per CU, and load the next transform while they
-// work on the current one (why, see product.hpp).  FFNT N = 2^16, 512
-// transforms: 127 -> 95 us (4.2 -> 5.7 TB/s in and out); R_R of 2^16 points, 128
-// transforms: 60 -> 50 us, against one workgroup per sub-problem with its
-// gather, LDS steps and stores one after the other.  The L2's repeated reads
-// bound it: R_R of 2^14 points, read twice instead of eight times, 1024
-// transforms: 94 -> 62 us (6.5 TB/s).
+// work on the current one (why, see product.hpp).  Against one workgroup per
+// sub-problem with its gather, LDS steps and stores one after the other, us, on
+// one buffer pair repeated and on pairs cycled beyond the last-level cache: FFNT
+// N = 2^16, 512 transforms (512 MiB in and out) 132 -> 101, 152 -> 134 (4.0
+// TB/s); R_R of 2^16 points x 128 61 -> 51, 61 -> 61; R_R of 2^14 points x 1024,
+// read twice instead of eight times, 94 -> 64, 94 -> 66 (6.1 TB/s).  Where the
+// product flow gains: persistent_forward, transform.hpp.
 #pragma once
 
 #include "oneshot.hpp"

@@ -35,10 +35,13 @@
 //   * geometry is compile-time, so addresses are one base per thread plus
 //     constants (XOR constants in LDS).
 // Measured against run-time geometry with every element through LDS first and
-// a table load per twiddle, forward us per call:
-//   FP64  2^13 x 1  14.2 -> 11.0    2^15 x 128  76 -> 41    2^23 x 1  196 -> 100
-//   FP32  2^13 x 1  11.4 ->  7.5    2^16 x  64  58 -> 24    2^20 x 8  115 -> 44
-//   special FP64  2^15 x 512  242 -> 136 (3.9 TB/s over its two passes)
+// a table load per twiddle, forward us per call on one buffer repeated, and on
+// buffers cycled beyond the last-level cache:
+//   FP64  2^13 x 1  14.4 -> 11.2          2^15 x 128  77 -> 41, 79 -> 56
+//         2^23 x 1  198 -> 100, 214 -> 136
+//   FP32  2^13 x 1  11.5 ->  7.7          2^16 x  64  60 -> 24, 65 -> 31
+//         2^20 x 8  114 -> 43, 119 -> 55
+//   special FP64  2^15 x 512  241 -> 135, 275 -> 166 (6.5 TB/s over its two passes)
 // Radix steps of at most 3 bits (one more exchange at 8 and 12 bits) were 2-10%
 // slower throughout.
 #pragma once

@@ -33,12 +33,13 @@
 // for life, those of the lowest step in vector registers, the uniform ones of
 // the top steps in scalar registers, and the rest in a small LDS table.
 //
-// Measured (us per call; before: one workgroup per product or sub-problem with
-// every step through LDS behind barriers, a table load per twiddle stage):
-//   ring 2^7  x 4096  54.5 -> 8.3     ring 2^12 x 2000  48.3 -> 40.1
-//   ring 2^13 x 1     17.0 -> 12.1    ring 2^13 x 1000  60.0 -> 43.4 (4.5 TB/s)
-//   ring 2^14 x 331   58.8 -> 48.7    ring 2^14 x 1000  138.7 -> 98.9 (4.0 TB/s)
-//   ring 2^16 x 256   132 -> 99.6 and the combine 47 (5.7 TB/s)
+// Measured (us per call on one set of buffers repeated, and on sets cycled
+// beyond the last-level cache; before: one workgroup per product or sub-problem
+// with every step through LDS behind barriers, a table load per twiddle stage):
+//   ring 2^7  x 4096  54.8 -> 8.3, 57.9 -> 9.4     ring 2^12 x 2000  50 -> 42, 60 -> 48
+//   ring 2^13 x 1     17.1 -> 12.1, 19.4 -> 12.4   ring 2^13 x 1000  62 -> 44, 73 -> 53 (3.7 TB/s)
+//   ring 2^14 x 331   59 -> 49, 65 -> 54           ring 2^14 x 1000  141 -> 100, 139 -> 100 (3.9 TB/s)
+//   ring 2^16 x 256   133 -> 103, 156 -> 122, and the combine 44 (6.1 TB/s)
 // Of that, at ring 2^14 x 1000: merged twiddles, registers and wavefront-local
 // exchanges 119, loads ahead 106, lane swaps 99.  At 2^13 points three LDS
 // exchanges and a table load per step spilled or stalled every variant.

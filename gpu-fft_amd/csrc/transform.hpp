@@ -24,8 +24,9 @@ struct PassPlan {
 // [0, K0) and column passes above it (pass.hpp).  One row pass up to 13 bits;
 // two passes to 2^24: 8 column bits keep 128-byte column rows and two radix
 // steps, and the row pass takes the rest, up to the 12 bits of the 2^12 tile;
-// beyond 2^20 the column pass grows too.  (FP64, 2^23 points, batch 1: 100 us
-// in 2 passes, 5.4 TB/s, against 197 us in 3 passes of at most 12 + 8 bits.)
+// beyond 2^20 the column pass grows too.  (FP64, 2^23 points, batch 1, against
+// 3 passes of at most 12 + 8 bits: 198 -> 100 us on one buffer, which the
+// last-level cache half holds, 214 -> 136 us (3.9 TB/s) on cycled ones.)
 // reversed: the CKKS passes read or write the row pass's tile in natural
 // order, which needs 2^(12-K0) >= 16 blocks for 128-byte runs, so K0 <= 8.
 inline std::vector<PassPlan> plan_passes(int n, bool descending, bool reversed)

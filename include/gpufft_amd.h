@@ -9,6 +9,9 @@
  * memory in the layouts of the reference library (Alisah-Ozcan/GPU-FFT):
  * complex values are interleaved (re, im) pairs of float (8 bytes) or
  * double (16 bytes), as COMPLEX<T> in src/include/gpufft/complex.cuh:14-16.
+ * A root table holds the powers of one primitive root, any one of either
+ * direction, in the layout that its function names; kernels derive some of its
+ * entries from others (quarter turns, products).
  *
  * The C++ templates of include/gpufft/fft.cuh (the reference's public
  * interface) are inline wrappers over these functions.
